@@ -52,10 +52,11 @@ def _case(name=None, kind="full", n=0, trajs=0, layout="aos", precision="fp32", 
 
 def listed():
     return [
-        # one MPC trajectory of 128 knots per call, the reference harness's size: latency
-        _case("call_128", n=128),
-        # the same from host memory to host memory (the reference's "GPU compute + I/O")
+        # one MPC trajectory of 128 knots, the reference harness's size, from host
+        # memory to host memory (its "GPU compute + I/O"): latency
         _case("host_128", kind="host", n=128),
+        # a few controllers' trajectories on the device in one call: latency
+        _case("call_2500", n=2500),
         # 64 solvers' trajectories of uneven length in one launch
         _case("batch_64", kind="batch", trajs=64),
         # a sampling controller's knots, an odd count below one wave per SIMD of 16-knot groups
@@ -218,6 +219,8 @@ def prepare(case, seed):
             s["vol"].t[:, 21:28] = d["qdd"]
         else:
             s["vol"] = _Dev(torch.cat([x, d["qdd"]], 1).contiguous())
+    if kind != "host":
+        s["result"] = _outputs(s)
     return s
 
 
@@ -229,6 +232,28 @@ def _pair(t):
     return {"dq": t[:, 0:49], "dqd": t[:, 49:98]}
 
 
+def _outputs(s):
+    """The output buffers of a state as named blocks, views made once."""
+    kind = s["kind"]
+    o = s["out"].t if "out" in s else None
+    if kind == "wafr":
+        return {"qdd": s["qdd"].t, "dqdd_dq": o[:, 0:49], "dqdd_dqd": o[:, 49:98], "minv": o[:, 98:147]}
+    if kind == "fd":
+        return {"qdd": s["qdd"].t, "minv": s["minv"].t}
+    if kind == "ref":
+        return _pair(o)
+    if kind in ("split", "fused"):
+        r = {"dtau": _pair(s["cdu"].t), "dqdd": _pair(o)}
+        if kind == "split":
+            v = s["vol"].t
+            r.update(v=v[:, 28:70], a=v[:, 70:112], f=v[:, 112:154])
+        return r
+    r = _blocks(o, 0 if "soa" in s else 1)
+    if kind == "minv":
+        r["minv"] = s["minv"].t
+    return r
+
+
 def run(s):
     kind, n, ctx = s["kind"], s["n"], s["ctx"]
     if kind == "host":
@@ -237,39 +262,28 @@ def run(s):
     if kind == "full":
         if "soa" in s:
             ctx.fdgrad_soa(n, s["in"], n, s["out"], n)
-            return _blocks(s["out"].t, 0)
-        ctx.fdgrad(n, s["in"], s["out"])
-        return _blocks(s["out"].t, 1)
-    if kind == "batch":
+        else:
+            ctx.fdgrad(n, s["in"], s["out"])
+    elif kind == "batch":
         s["batch"].run(s["trajs"])
-        return _blocks(s["out"].t, 1)
-    if kind == "minv":
+    elif kind == "minv":
         ctx.fdgrad_minv(n, s["in"], s["out"], s["minv"])
-        return dict(_blocks(s["out"].t, 1), minv=s["minv"].t)
-    if kind == "wafr":
+    elif kind == "wafr":
         ctx.fdgrad_wafr(n, s["in"], s["qdd"], s["out"])
-        o = s["out"].t
-        return {"qdd": s["qdd"].t, "dqdd_dq": o[:, 0:49], "dqdd_dqd": o[:, 49:98], "minv": o[:, 98:147]}
-    if kind == "fext":
+    elif kind == "fext":
         ctx.fdgrad_fext(n, s["in"], s["fext"], 42, s["out"])
-        return _blocks(s["out"].t, 1)
-    if kind == "ref":
+    elif kind == "ref":
         ctx.dynamics_gradient_kernel(n, s["out"], s["vol"])
-        return _pair(s["out"].t)
-    if kind == "fd":
+    elif kind == "fd":
         ctx.forward_dynamics_dev(n, s["in"], s["qdd"], s["minv"])
-        return {"qdd": s["qdd"].t, "minv": s["minv"].t}
-    if kind == "split":
-        ctx.gradient_setup_split_dev(n, s["vol"])
-        ctx.dynamics_gradient_kernel_split(n, s["cdu"], s["vol"])
     else:
-        ctx.dynamics_gradient_kernel_fused(n, s["cdu"], s["vol"])
-    ctx.gradient_finish_dev(n, s["out"], s["cdu"], s["minv"])
-    r = {"dtau": _pair(s["cdu"].t), "dqdd": _pair(s["out"].t)}
-    if kind == "split":
-        v = s["vol"].t
-        r.update(v=v[:, 28:70], a=v[:, 70:112], f=v[:, 112:154])
-    return r
+        if kind == "split":
+            ctx.gradient_setup_split_dev(n, s["vol"])
+            ctx.dynamics_gradient_kernel_split(n, s["cdu"], s["vol"])
+        else:
+            ctx.dynamics_gradient_kernel_fused(n, s["cdu"], s["vol"])
+        ctx.gradient_finish_dev(n, s["out"], s["cdu"], s["minv"])
+    return s["result"]
 
 
 # ---------------------------------------------------------------------------
