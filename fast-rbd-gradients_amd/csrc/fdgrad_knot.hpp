@@ -58,6 +58,9 @@ RBD_HD RBD_INLINE void static_for_down(F&& f) {
 
 template <typename S> struct CS { S c, s; };
 
+RBD_HD RBD_INLINE float fma_s(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+RBD_HD RBD_INLINE double fma_s(double a, double b, double c) { return __builtin_fma(a, b, c); }
+
 RBD_HD RBD_INLINE void sincos_s(float x, float* s, float* c) {
 #if defined(__HIP_DEVICE_COMPILE__)
   ::sincosf(x, s, c);
@@ -201,63 +204,166 @@ RBD_HD RBD_INLINE void crf(const S* x, const S* z, S* y) {
 }
 
 // ---------------------------------------------------------------------------
-// Articulated-inertia transport: P = T^T Ia T for a symmetric Ia whose row and
-// column 2 are zero (revolute joint about z).  T = [E 0; 0 E][1 0; -r^ 1]:
-// rotate the 3x3 blocks (A' = E^T A E, C' = E^T C E, M' = E^T M E), then
-// translate: TL = A' + r^ C'^T - C' r^ - r^ M' r^, TR = C' + r^ M', BR = M'.
-// (Same product as the reference's ctransform_Ia_revolute, minv.h:221-386.)
+// The recursions below are written with every multiply-add explicit (fma_s),
+// so that each kernel that inlines them computes bitwise the same values: left
+// to the compiler, which product of a sum is fused differs from kernel to
+// kernel.  Products with structural zeros still fold away.
 // ---------------------------------------------------------------------------
+// F of E = Z(q) F, Z = [c s 0; -s c 0; 0 0 1]: the joint's fixed rotation
+template <int K>
+RBD_HD constexpr double fixed_rot(int i, int j) {
+  return i < 2 ? double(ecoef_c(K, i, j)) : double(ecoef_1(K, 2, j));
+}
+template <int K>
+RBD_HD constexpr bool signed_permutation() {
+  for (int i = 0; i < 3; ++i)
+    for (int j = 0; j < 3; ++j) {
+      const double f = fixed_rot<K>(i, j);
+      if (f != 0.0 && f != 1.0 && f != -1.0) return false;
+    }
+  return true;
+}
+template <typename S, int K, int I, int J> constexpr S kFixed = S(fixed_rot<K>(I, J));
+
+// (F^T x)_J and (F x)_I
+template <int K, int J, typename S>
+RBD_HD RBD_INLINE S fixed_t(const S* x) {
+  return fma_s(kFixed<S, K, 0, J>, x[0], fma_s(kFixed<S, K, 1, J>, x[1], kFixed<S, K, 2, J> * x[2]));
+}
+template <int K, int I, typename S>
+RBD_HD RBD_INLINE S fixed(const S* x) {
+  return fma_s(kFixed<S, K, I, 0>, x[0], fma_s(kFixed<S, K, I, 1>, x[1], kFixed<S, K, I, 2> * x[2]));
+}
+// y = E x
 template <int K, typename S>
-RBD_HD RBD_INLINE void transport(const CS<S>& t, const S Ia[6][6], S P[6][6]) {
-  S A[3][3], C[3][3], M[3][3];
-  for (int i = 0; i < 3; ++i)
-    for (int j = 0; j < 3; ++j) { A[i][j] = Ia[i][j]; C[i][j] = Ia[i][j + 3]; M[i][j] = Ia[i + 3][j + 3]; }
-  // X' = E^T X E : first Y = X E (rows of X times E), then E^T Y
-  auto sandwich = [&](const S X[3][3], S out[3][3]) {
-    S Y[3][3];
-    for (int i = 0; i < 3; ++i) {
-      S row_e[3];
-      // (X E)[i][j] = sum_l X[i][l] E[l][j] = (E^T x_i)_j  with x_i the i-th row
-      const S xi[3] = {X[i][0], X[i][1], X[i][2]};
-      rot_t<K>(t, xi, row_e);
-      Y[i][0] = row_e[0]; Y[i][1] = row_e[1]; Y[i][2] = row_e[2];
-    }
-    for (int j = 0; j < 3; ++j) {
-      const S yj[3] = {Y[0][j], Y[1][j], Y[2][j]};
-      S col[3];
-      rot_t<K>(t, yj, col);            // (E^T Y)[:, j] = E^T y_j
-      out[0][j] = col[0]; out[1][j] = col[1]; out[2][j] = col[2];
-    }
-  };
-  S Ar[3][3], Cr[3][3], Mr[3][3];
-  sandwich(A, Ar);
-  sandwich(C, Cr);
-  sandwich(M, Mr);
+RBD_HD RBD_INLINE void to_child(const CS<S>& t, const S* x, S* y) {
+  const S w0 = fixed<K, 0>(x), w1 = fixed<K, 1>(x), w2 = fixed<K, 2>(x);
+  y[0] = fma_s(t.s, w1, t.c * w0);
+  y[1] = fma_s(-t.s, w0, t.c * w1);
+  y[2] = w2;
+}
+// y = E^T x, and y = E^T x + z
+template <int K, typename S>
+RBD_HD RBD_INLINE void to_parent(const CS<S>& t, const S* x, S* y) {
+  const S w[3] = {fma_s(-t.s, x[1], t.c * x[0]), fma_s(t.s, x[0], t.c * x[1]), x[2]};
+  const S y0 = fixed_t<K, 0>(w), y1 = fixed_t<K, 1>(w), y2 = fixed_t<K, 2>(w);
+  y[0] = y0; y[1] = y1; y[2] = y2;
+}
+template <int K, typename S>
+RBD_HD RBD_INLINE void to_parent_add(const CS<S>& t, const S* x, const S* z, S* y) {
+  if constexpr (signed_permutation<K>()) {
+    // F^T (Z^T x + F z): the permuted z starts the sums, two adds fewer
+    const S w[3] = {fma_s(-t.s, x[1], fma_s(t.c, x[0], fixed<K, 0>(z))),
+                    fma_s(t.s, x[0], fma_s(t.c, x[1], fixed<K, 1>(z))), x[2] + fixed<K, 2>(z)};
+    const S y0 = fixed_t<K, 0>(w), y1 = fixed_t<K, 1>(w), y2 = fixed_t<K, 2>(w);
+    y[0] = y0; y[1] = y1; y[2] = y2;
+  } else {
+    S w[3];
+    to_parent<K>(t, x, w);
+    y[0] = z[0] + w[0]; y[1] = z[1] + w[1]; y[2] = z[2] + w[2];
+  }
+}
+// y += r x f, r joint K's offset
+template <int K, typename S>
+RBD_HD RBD_INLINE void add_offset_cross(const S* f, S* y) {
   constexpr S rx = roff<K, S>(0), ry = roff<K, S>(1), rz = roff<K, S>(2);
-  const S R[3][3] = {{S(0), -rz, ry}, {rz, S(0), -rx}, {-ry, rx, S(0)}};
-  // TR = Cr + R Mr
-  S TR[3][3], RM[3][3];
-  for (int i = 0; i < 3; ++i)
-    for (int j = 0; j < 3; ++j) {
-      RM[i][j] = R[i][0] * Mr[0][j] + R[i][1] * Mr[1][j] + R[i][2] * Mr[2][j];
-      TR[i][j] = Cr[i][j] + RM[i][j];
-    }
-  // TL = Ar + R Cr^T - Cr R - R Mr R = Ar + R Cr^T - (Cr + R Mr) R = Ar + R Cr^T - TR R
-  for (int i = 0; i < 3; ++i)
-    for (int j = 0; j <= i; ++j) {
-      const S rct = R[i][0] * Cr[j][0] + R[i][1] * Cr[j][1] + R[i][2] * Cr[j][2];
-      const S trr = TR[i][0] * R[0][j] + TR[i][1] * R[1][j] + TR[i][2] * R[2][j];
-      const S e = Ar[i][j] + rct - trr;
-      P[i][j] = e; P[j][i] = e;
-    }
-  for (int i = 0; i < 3; ++i)
-    for (int j = 0; j < 3; ++j) {
-      P[i][j + 3] = TR[i][j];
-      P[j + 3][i] = TR[i][j];
-      P[i + 3][j + 3] = Mr[i][j];
-    }
+  y[0] = fma_s(ry, f[2], fma_s(-rz, f[1], y[0]));
+  y[1] = fma_s(rz, f[0], fma_s(-rx, f[2], y[1]));
+  y[2] = fma_s(rx, f[1], fma_s(-ry, f[0], y[2]));
+}
+// x = T x for a motion vector (parent to child), in place
+template <int K, typename S>
+RBD_HD RBD_INLINE void move_motion(const CS<S>& t, const S* x, S* y) {
+  constexpr S rx = roff<K, S>(0), ry = roff<K, S>(1), rz = roff<K, S>(2);
+  const S d[3] = {fma_s(-ry, x[2], fma_s(rz, x[1], x[3])), fma_s(-rz, x[0], fma_s(rx, x[2], x[4])),
+                  fma_s(-rx, x[1], fma_s(ry, x[0], x[5]))};
+  S w[3];
+  to_child<K>(t, x, w);
+  to_child<K>(t, d, y + 3);
+  y[0] = w[0]; y[1] = w[1]; y[2] = w[2];
+}
+// x = T^T x for a force vector (child to parent), in place
+template <int K, typename S>
+RBD_HD RBD_INLINE void move_force(const CS<S>& t, S* x) {
+  to_parent<K>(t, x, x);
+  to_parent<K>(t, x + 3, x + 3);
+  add_offset_cross<K>(x + 3, x);
+}
+// z += T^T x
+template <int K, typename S>
+RBD_HD RBD_INLINE void add_moved_force(const CS<S>& t, const S* x, S* z) {
+  S f[3];
+  to_parent<K>(t, x + 3, f);
+  to_parent_add<K>(t, x, z, z);
+  add_offset_cross<K>(f, z);
+  z[3] += f[0]; z[4] += f[1]; z[5] += f[2];
+}
+// y = I_K x, I_K the constant inertia of link K
+template <int K, typename S>
+RBD_HD RBD_INLINE void inertia_times(const S* x, S* y) {
+  static_for<0, 6>([&](auto Rc) {
+    constexpr int r = decltype(Rc)::value;
+    S acc = kInertia<S, K, r, 0> * x[0];
+    static_for<1, 6>([&](auto Cc) {
+      constexpr int c = decltype(Cc)::value;
+      acc = fma_s(kInertia<S, K, r, c>, x[c], acc);
+    });
+    y[r] = acc;
+  });
+}
+// y += x x* z
+template <typename S>
+RBD_HD RBD_INLINE void add_force_cross(const S* x, const S* z, S* y) {
+  y[0] = fma_s(x[1], z[2], fma_s(-x[2], z[1], fma_s(x[4], z[5], fma_s(-x[5], z[4], y[0]))));
+  y[1] = fma_s(x[2], z[0], fma_s(-x[0], z[2], fma_s(x[5], z[3], fma_s(-x[3], z[5], y[1]))));
+  y[2] = fma_s(x[0], z[1], fma_s(-x[1], z[0], fma_s(x[3], z[4], fma_s(-x[4], z[3], y[2]))));
+  y[3] = fma_s(x[1], z[5], fma_s(-x[2], z[4], y[3]));
+  y[4] = fma_s(x[2], z[3], fma_s(-x[0], z[5], y[4]));
+  y[5] = fma_s(x[0], z[4], fma_s(-x[1], z[3], y[5]));
 }
 
+// Symmetric 3x3 matrices are stored as xx, xy, xz, yy, yz, zz.
+RBD_HD constexpr int sym(int i, int j) { return (i == 0 || j == 0) ? i + j : i + j + 1; }
+// products of a joint's sin and cos: sin^2 q, sin 2q, cos 2q, sin(2q) / 2
+template <typename S> struct DoubleAngle { S ss, s2, c2, sc; };
+template <typename S>
+RBD_HD RBD_INLINE DoubleAngle<S> double_angle(const CS<S>& t) {
+  const S ss = t.s * t.s, sc = t.c * t.s;
+  return {ss, sc + sc, fma_s(S(-2), ss, S(1)), sc};
+}
+// A = E^T A E.  The z rotation leaves the trace of the x-y block, so the block
+// takes 7 operations instead of the 14 of two one-sided rotations.
+template <int K, typename S>
+RBD_HD RBD_INLINE void sym_to_parent(const CS<S>& t, const DoubleAngle<S>& q, S A[6]) {
+  const S d = A[3] - A[0];
+  const S e = fma_s(-q.s2, A[1], q.ss * d);
+  const S B[6] = {A[0] + e, fma_s(-q.sc, d, q.c2 * A[1]), fma_s(-t.s, A[4], t.c * A[2]),
+                  A[3] - e, fma_s(t.s, A[2], t.c * A[4]), A[5]};
+  static_for<0, 3>([&](auto Ic) {
+    constexpr int i = decltype(Ic)::value;
+    S col[3];                                    // column i of B F
+    static_for<0, 3>([&](auto Rc) {
+      constexpr int r = decltype(Rc)::value;
+      const S row[3] = {B[sym(r, 0)], B[sym(r, 1)], B[sym(r, 2)]};
+      col[r] = fixed_t<K, i>(row);
+    });
+    static_for<0, i + 1>([&](auto Jc) {
+      constexpr int j = decltype(Jc)::value;
+      A[sym(j, i)] = fixed_t<K, j>(col);
+    });
+  });
+}
+// A += g (2 (r.h) 1 - h r^T - r h^T)
+template <typename S>
+RBD_HD RBD_INLINE void add_sym_outer(S g, S rx, S ry, S rz, const S* h, S A[6]) {
+  const S gx = g * rx, gy = g * ry, gz = g * rz;
+  A[0] = fma_s(S(2) * gy, h[1], fma_s(S(2) * gz, h[2], A[0]));
+  A[3] = fma_s(S(2) * gx, h[0], fma_s(S(2) * gz, h[2], A[3]));
+  A[5] = fma_s(S(2) * gx, h[0], fma_s(S(2) * gy, h[1], A[5]));
+  A[1] = fma_s(-gx, h[1], fma_s(-gy, h[0], A[1]));
+  A[2] = fma_s(-gx, h[2], fma_s(-gz, h[0], A[2]));
+  A[4] = fma_s(-gy, h[2], fma_s(-gz, h[1], A[4]));
+}
 
 // ---------------------------------------------------------------------------
 // Arithmetic precision per phase.  Inputs and outputs are FP32 in every mode.
@@ -313,153 +419,211 @@ RBD_HD RBD_INLINE void knot_sincos(S x, S* s, S* c) {
 }
 
 // ---------------------------------------------------------------------------
-// Minv = M^-1 (upper triangle, Mi[r][c] for r <= c) by the articulated-body
-// recursion (computeMinv, minv.h:423-478; equation numbers as in its comments).
+// The mass matrix in factors, M = L^T D L with L unit lower triangular, from the
+// articulated-body recursion: D_k = S^T IA_k S, the pivots of computeMinv
+// (minv.h:423-478), and L[k][j] = S_j^T (IA_k S / D_k moved to link j).  A
+// right-hand side costs the 49 multiply-adds of a product with Minv, and the
+// recursion has neither the F columns nor the forward pass that forming Minv
+// takes (about 700 instructions against 1,300); factoring the joint-space
+// matrix from composite inertias would take fewer still but doubled the error
+// of dqdd/dq (4.7e-7 against 2.2e-7 in FP32).
 // The pivots D_k and 1/D_k are formed in SP (FP64 in the pivot variant).
 // ---------------------------------------------------------------------------
+template <typename S> struct MassFactors {
+  S L[NQ][NQ];     // [k][j], j < k
+  S dinv[NQ];
+};
+
+// 1 / x of a pivot
+RBD_HD RBD_INLINE float reciprocal(float x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const float r = __builtin_amdgcn_rcpf(x);      // within one unit in the last place; a Newton step
+  return __builtin_fmaf(__builtin_fmaf(-x, r, 1.0f), r, r);
+#else
+  return 1.0f / x;
+#endif
+}
+RBD_HD RBD_INLINE double reciprocal(double x) { return 1.0 / x; }
+
+// T^T Ia T of a symmetric Ia = [A C; C^T N] whose row and column 2 are zero (a
+// revolute joint about z): A = (xx, xy, yy), C rows 0 and 1, N all six.  The
+// 3x3 blocks are rotated (A' = E^T A E, C' = E^T C E, N' = E^T N E), then
+// translated: TR = C' + r^ N', TL = A' + r^ C'^T - TR r^, BR = N'.
+// (Same product as the reference's ctransform_Ia_revolute, minv.h:221-386.)
+template <int K, typename S>
+RBD_HD RBD_INLINE void move_articulated(const CS<S>& t, const S a[3], const S c[2][3], const S n[6], S TL[6],
+                                        S TR[3][3], S BR[6]) {
+  const DoubleAngle<S> q = double_angle(t);
+  TL[0] = a[0]; TL[1] = a[1]; TL[3] = a[2]; TL[2] = S(0); TL[4] = S(0); TL[5] = S(0);
+  sym_to_parent<K>(t, q, TL);
+  for (int i = 0; i < 6; ++i) BR[i] = n[i];
+  sym_to_parent<K>(t, q, BR);
+  S r0[3], r1[3], C[3][3];                       // C E, then E^T (C E)
+  to_parent<K>(t, c[0], r0);
+  to_parent<K>(t, c[1], r1);
+  static_for<0, 3>([&](auto Jc) {
+    constexpr int j = decltype(Jc)::value;
+    const S col[3] = {r0[j], r1[j], S(0)};
+    S y[3];
+    to_parent<K>(t, col, y);
+    C[0][j] = y[0]; C[1][j] = y[1]; C[2][j] = y[2];
+    const S b[3] = {BR[sym(0, j)], BR[sym(1, j)], BR[sym(2, j)]};
+    add_offset_cross<K>(b, y);
+    TR[0][j] = y[0]; TR[1][j] = y[1]; TR[2][j] = y[2];
+  });
+  // (r^ C'^T)_ij = (r x C'_j)_i, (TR r^)_ij = -(r x TR_i)_j, rows of C' and TR
+  static_for<0, 3>([&](auto Ic) {
+    constexpr int i = decltype(Ic)::value;
+    static_for<i, 3>([&](auto Jc) {
+      constexpr int j = decltype(Jc)::value;
+      constexpr int i1 = (i + 1) % 3, i2 = (i + 2) % 3, j1 = (j + 1) % 3, j2 = (j + 2) % 3;
+      TL[sym(i, j)] = fma_s(roff<K, S>(i1), C[j][i2], fma_s(-roff<K, S>(i2), C[j][i1],
+                      fma_s(roff<K, S>(j1), TR[i][j2], fma_s(-roff<K, S>(j2), TR[i][j1], TL[sym(i, j)]))));
+    });
+  });
+}
+
 template <typename S, typename SP>
-RBD_HD RBD_INLINE void compute_minv(const CS<S>* t, S Mi[NQ][NQ]) {
-  S IA[6][6];
-  SP IA22;                    // IA[2][2] (the pivot) carried in SP
-  iload<NQ - 1>(IA);
-  IA22 = SP(IA[2][2]);
-  S F[NQ][6];                 // F[j] = F_k[:, j], columns j >= k meaningful
-  S U[NQ][6], Dinv[NQ];
-  for (int j = 0; j < NQ; ++j)
-    for (int r = 0; r < 6; ++r) F[j][r] = S(0);
+RBD_HD RBD_INLINE void mass_factors(const CS<S>* t, MassFactors<S>& f) {
+  // articulated inertia of link k: [A C; C^T N]
+  S A[6], C[3][3], N[6];
+  static_for<0, 3>([&](auto Ic) {
+    constexpr int i = decltype(Ic)::value;
+    static_for<0, 3>([&](auto Jc) {
+      constexpr int j = decltype(Jc)::value;
+      C[i][j] = kInertia<S, NQ - 1, i, 3 + j>;
+      if constexpr (j >= i) {
+        A[sym(i, j)] = kInertia<S, NQ - 1, i, j>;
+        N[sym(i, j)] = kInertia<S, NQ - 1, 3 + i, 3 + j>;
+      }
+    });
+  });
+  SP pivot = SP(kInertia<S, NQ - 1, 2, 2>);
   static_for_down<NQ, 0>([&](auto Kc) {
     constexpr int k = decltype(Kc)::value;
-    for (int r = 0; r < 6; ++r) U[k][r] = IA[r][2];        // U = IA S
-    const SP dinv = SP(1) / IA22;                            // 1 / (S^T IA S)
-    Dinv[k] = S(dinv);
-    Mi[k][k] = Dinv[k];                                      // (21)
-    static_for<k + 1, NQ>([&](auto Jc) {                     // (12)
-      constexpr int j = decltype(Jc)::value;
-      Mi[k][j] = -Dinv[k] * F[j][2];
-    });
-    static_for<k, NQ>([&](auto Jc) {                         // (14), (19)
-      constexpr int j = decltype(Jc)::value;
-      for (int r = 0; r < 6; ++r) F[j][r] += U[k][r] * Mi[k][j];
-    });
+    f.dinv[k] = S(reciprocal(pivot));
     if constexpr (k > 0) {
-      static_for<k, NQ>([&](auto Jc) {                       // (15): F_{k-1} = T^T F_k
+      const S U[6] = {A[2], A[4], A[5], C[2][0], C[2][1], C[2][2]};      // IA S
+      S W[6];                                                              // U / D
+      for (int i = 0; i < 6; ++i) W[i] = i == 2 ? S(1) : U[i] * f.dinv[k];
+      // IA - U U^T / D
+      const S a[3] = {fma_s(-U[0], W[0], A[0]), fma_s(-U[0], W[1], A[1]), fma_s(-U[1], W[1], A[3])};
+      S c[2][3], n[6];
+      static_for<0, 3>([&](auto Jc) {
         constexpr int j = decltype(Jc)::value;
-        S y[6];
-        xforce_t<k>(t[k], F[j], y);
-        for (int r = 0; r < 6; ++r) F[j][r] = y[r];
+        c[0][j] = fma_s(-U[0], W[3 + j], C[0][j]);
+        c[1][j] = fma_s(-U[1], W[3 + j], C[1][j]);
+        static_for<0, j + 1>([&](auto Ic) {
+          constexpr int i = decltype(Ic)::value;
+          n[sym(i, j)] = fma_s(-U[3 + i], W[3 + j], N[sym(i, j)]);
+        });
       });
-      S Ia[6][6];                                            // IA - U U^T / D
-      S UD[6];
-      for (int r = 0; r < 6; ++r) UD[r] = U[k][r] * Dinv[k];
-      for (int r = 0; r < 6; ++r)
-        for (int c = 0; c < 6; ++c)
-          Ia[r][c] = (r == 2 || c == 2) ? S(0) : IA[r][c] - U[k][r] * UD[c];
-      S P[6][6];
-      transport<k>(t[k], Ia, P);
-      iload<k - 1>(IA);
-      for (int r = 0; r < 6; ++r)
-        for (int c = 0; c < 6; ++c) IA[r][c] += P[r][c];
+      S TL[6], TR[3][3], BR[6];
+      move_articulated<k>(t[k], a, c, n, TL, TR, BR);
+      static_for<0, 3>([&](auto Ic) {
+        constexpr int i = decltype(Ic)::value;
+        static_for<0, 3>([&](auto Jc) {
+          constexpr int j = decltype(Jc)::value;
+          C[i][j] = TR[i][j] + kInertia<S, k - 1, i, 3 + j>;
+          if constexpr (j >= i) {
+            A[sym(i, j)] = TL[sym(i, j)] + kInertia<S, k - 1, i, j>;
+            N[sym(i, j)] = BR[sym(i, j)] + kInertia<S, k - 1, 3 + i, 3 + j>;
+          }
+        });
+      });
       if constexpr (sizeof(SP) > sizeof(S)) {
-        // the next pivot S^T IA_{k-1} S formed in SP from the same (rounded) terms;
-        // only entry (2,2) of this second transport is live, the rest is dead code
-        SP IaW[6][6], PW[6][6];
-        for (int r = 0; r < 6; ++r)
-          for (int c = 0; c < 6; ++c) IaW[r][c] = SP(Ia[r][c]);
+        // the next pivot formed in SP from the same (rounded) terms; only
+        // entry (2, 2) of this second transport is live, the rest is dead code
+        const SP aw[3] = {SP(a[0]), SP(a[1]), SP(a[2])};
+        SP cw[2][3], nw[6], TLw[6], TRw[3][3], BRw[6];
+        for (int j = 0; j < 3; ++j) { cw[0][j] = SP(c[0][j]); cw[1][j] = SP(c[1][j]); }
+        for (int i = 0; i < 6; ++i) nw[i] = SP(n[i]);
         const CS<SP> tw{SP(t[k].c), SP(t[k].s)};
-        transport<k>(tw, IaW, PW);
-        IA22 = SP(inertia_entry(k - 1, 2, 2)) + PW[2][2];
+        move_articulated<k>(tw, aw, cw, nw, TLw, TRw, BRw);
+        pivot = SP(inertia_entry(k - 1, 2, 2)) + TLw[5];
       } else {
-        IA22 = SP(IA[2][2]);
+        pivot = SP(A[5]);
       }
-    }
-  });
-  // forward pass (Minv_fp, minv.h:439-469): F_k[:, j] = S Minv[k, j] + T F_{k-1}[:, j]
-  static_for<0, NQ>([&](auto Kc) {
-    constexpr int k = decltype(Kc)::value;
-    if constexpr (k == 0) {
-      for (int j = 0; j < NQ; ++j) {
-        for (int r = 0; r < 6; ++r) F[j][r] = S(0);
-        F[j][2] = Mi[0][j];
-      }
-    } else {
-      static_for<k, NQ>([&](auto Jc) {
-        constexpr int j = decltype(Jc)::value;
-        S w[6];
-        xmotion<k>(t[k], F[j], w);                           // T F_{k-1}[:, j]
-        const S uw = U[k][0] * w[0] + U[k][1] * w[1] + U[k][2] * w[2] +
-                     U[k][3] * w[3] + U[k][4] * w[4] + U[k][5] * w[5];
-        Mi[k][j] -= Dinv[k] * uw;                            // (30)
-        w[2] += Mi[k][j];                                    // (32) + (34)
-        for (int r = 0; r < 6; ++r) F[j][r] = w[r];
+      static_for_down<k + 1, 1>([&](auto Jc) {
+        constexpr int j = decltype(Jc)::value;   // W from link j to link j - 1
+        move_force<j>(t[j], W);
+        f.L[k][j - 1] = W[2];
       });
     }
   });
 }
 
-// Column j of Minv, for a lane that computes one column: col[k] = Minv[k][j]
-// for k <= j (entries k > j are left unspecified).  The articulated inertias
-// (U_k, D_k, the IA transports) are computed in full, the F and Minv updates
-// for column j only -- the recursion of compute_minv restricted to one column.
-// Through the backward pass column j's F stays exactly zero for every link
-// k > j (its Minv entry there is -D_k^-1 * 0), so one code path serves every j.
+// x = M^-1 x (NEG: negated)
+template <bool NEG, typename S, typename SX>
+RBD_HD RBD_INLINE void mass_solve(const MassFactors<S>& f, SX x[NQ]) {
+  static_for_down<NQ, 1>([&](auto Kc) {
+    constexpr int k = decltype(Kc)::value;
+    static_for<0, k>([&](auto Jc) {
+      constexpr int j = decltype(Jc)::value;
+      x[j] = fma_s(-SX(f.L[k][j]), x[k], x[j]);
+    });
+  });
+  for (int k = 0; k < NQ; ++k) x[k] = (NEG ? -x[k] : x[k]) * SX(f.dinv[k]);
+  static_for<1, NQ>([&](auto Kc) {
+    constexpr int k = decltype(Kc)::value;
+    static_for<0, k>([&](auto Jc) {
+      constexpr int j = decltype(Jc)::value;
+      x[k] = fma_s(-SX(f.L[k][j]), x[j], x[k]);
+    });
+  });
+}
+
+// Column j of Minv from the factors: col[k] = Minv[k][j] for k <= j (the
+// entries below are formed too far only to k = j when J is a constant, and
+// left unspecified).  The forward sums of links k > j are exactly zero, so the
+// run-time j of the lane groups gives bitwise the entries of a constant j.
+template <int J, typename S>
+RBD_HD RBD_INLINE void minv_column(const MassFactors<S>& f, int j, S col[NQ]) {
+  constexpr int top = J < 0 ? NQ : J + 1;        // rows to form
+  S y[NQ];
+  static_for_down<top, 0>([&](auto Kc) {
+    constexpr int k = decltype(Kc)::value;
+    S acc = (J < 0 ? k == j : k == J) ? S(1) : S(0);
+    static_for_down<top, k + 1>([&](auto Ic) {
+      constexpr int i = decltype(Ic)::value;
+      acc = fma_s(-f.L[i][k], y[i], acc);
+    });
+    y[k] = acc;
+  });
+  static_for<0, top>([&](auto Kc) {
+    constexpr int k = decltype(Kc)::value;
+    S acc = y[k] * f.dinv[k];
+    static_for<0, k>([&](auto Ic) {
+      constexpr int i = decltype(Ic)::value;
+      acc = fma_s(-f.L[k][i], col[i], acc);
+    });
+    col[k] = acc;
+  });
+}
+
+// Minv (upper triangle, Mi[r][c] for r <= c)
+template <typename S>
+RBD_HD RBD_INLINE void minv_from_factors(const MassFactors<S>& f, S Mi[NQ][NQ]) {
+  static_for<0, NQ>([&](auto Jc) {
+    constexpr int j = decltype(Jc)::value;
+    S col[NQ];
+    minv_column<j>(f, j, col);
+    for (int r = 0; r <= j; ++r) Mi[r][j] = col[r];
+  });
+}
+template <typename S, typename SP>
+RBD_HD RBD_INLINE void compute_minv(const CS<S>* t, S Mi[NQ][NQ]) {
+  MassFactors<S> f;
+  mass_factors<S, SP>(t, f);
+  minv_from_factors(f, Mi);
+}
+// Column j of Minv, for a lane that computes one column (entries k > j are
+// left unspecified).
 template <typename S, typename SP>
 RBD_HD RBD_INLINE void compute_minv_column(const CS<S>* t, int j, S col[NQ]) {
-  S IA[6][6];
-  SP IA22;
-  iload<NQ - 1>(IA);
-  IA22 = SP(IA[2][2]);
-  S F[6] = {S(0), S(0), S(0), S(0), S(0), S(0)};
-  S U[NQ][6], Dinv[NQ];
-  static_for_down<NQ, 0>([&](auto Kc) {
-    constexpr int k = decltype(Kc)::value;
-    for (int r = 0; r < 6; ++r) U[k][r] = IA[r][2];
-    const SP dinv = SP(1) / IA22;
-    Dinv[k] = S(dinv);
-    col[k] = (j == k) ? Dinv[k] : -Dinv[k] * F[2];          // (21), (12)
-    for (int r = 0; r < 6; ++r) F[r] += U[k][r] * col[k];   // (14), (19)
-    if constexpr (k > 0) {
-      S y[6];
-      xforce_t<k>(t[k], F, y);                               // (15)
-      for (int r = 0; r < 6; ++r) F[r] = y[r];
-      S Ia[6][6];
-      S UD[6];
-      for (int r = 0; r < 6; ++r) UD[r] = U[k][r] * Dinv[k];
-      for (int r = 0; r < 6; ++r)
-        for (int c = 0; c < 6; ++c)
-          Ia[r][c] = (r == 2 || c == 2) ? S(0) : IA[r][c] - U[k][r] * UD[c];
-      S P[6][6];
-      transport<k>(t[k], Ia, P);
-      iload<k - 1>(IA);
-      for (int r = 0; r < 6; ++r)
-        for (int c = 0; c < 6; ++c) IA[r][c] += P[r][c];
-      if constexpr (sizeof(SP) > sizeof(S)) {
-        SP IaW[6][6], PW[6][6];
-        for (int r = 0; r < 6; ++r)
-          for (int c = 0; c < 6; ++c) IaW[r][c] = SP(Ia[r][c]);
-        const CS<SP> tw{SP(t[k].c), SP(t[k].s)};
-        transport<k>(tw, IaW, PW);
-        IA22 = SP(inertia_entry(k - 1, 2, 2)) + PW[2][2];
-      } else {
-        IA22 = SP(IA[2][2]);
-      }
-    }
-  });
-  // forward pass: F_k = S Minv[k, j] + T F_{k-1}
-  static_for<0, NQ>([&](auto Kc) {
-    constexpr int k = decltype(Kc)::value;
-    if constexpr (k == 0) {
-      for (int r = 0; r < 6; ++r) F[r] = S(0);
-      F[2] = col[0];
-    } else {
-      S w[6];
-      xmotion<k>(t[k], F, w);
-      const S uw = U[k][0] * w[0] + U[k][1] * w[1] + U[k][2] * w[2] +
-                   U[k][3] * w[3] + U[k][4] * w[4] + U[k][5] * w[5];
-      col[k] -= Dinv[k] * uw;                                 // (30)
-      w[2] += col[k];                                         // (32) + (34)
-      for (int r = 0; r < 6; ++r) F[r] = w[r];
-    }
-  });
+  MassFactors<S> f;
+  mass_factors<S, SP>(t, f);
+  minv_column<-1>(f, j, col);
 }
 
 // ---------------------------------------------------------------------------
@@ -528,74 +692,92 @@ RBD_HD RBD_INLINE void subtract_fext(const In& in, S f[NQ][6]) {
 // Backward sweep (compute_cdu, :831-857): g_{k-1} = df_{k-1} + T^T g_k, with the
 // extra T^T (-(f_k x S)) at k == c for d/dq; dtau_k = g_k[2].
 // ---------------------------------------------------------------------------
+// Written per link instead of as a recursion in (dv, da): with
+// D_c = 2 v_c x S and P_c = a_c x S + v_c x (v_c x S), both moved to link k,
+//   d/dq_c:   df_k = I_k P_c + B_k D_c
+//   d/dqd_c:  df_k = I_k D_c + 2 B_k S
+// with B_k = ((v_k x*) I_k - I_k (v_k x) + (. x* h_k)) / 2, h_k = I_k v_k the
+// momentum.  B maps [w; u] to [(Bs - n^ / 2) w; -p x w] with Bs symmetric and
+// (n, p) the momentum, so it sees only the angular part of its argument: a
+// column takes 65 instructions a link and seed in place of 120, and its
+// largest error is about half (dqdd/dqd 4.9e-7 against 8.2e-7 of the norm).
+// first moment of link K (mass times centre of mass)
+template <int K>
+RBD_HD constexpr double first_moment(int i) {
+  return i == 0 ? inertia_entry(K, 2, 4) : (i == 1 ? inertia_entry(K, 0, 5) : inertia_entry(K, 1, 3));
+}
+// Bs of link K alone at velocity v
+template <int K, typename S>
+RBD_HD RBD_INLINE void body_bs(const S* v, S B[6]) {
+  constexpr double xx = inertia_entry(K, 0, 0), xy = inertia_entry(K, 0, 1), xz = inertia_entry(K, 0, 2),
+                   yy = inertia_entry(K, 1, 1), yz = inertia_entry(K, 1, 2), zz = inertia_entry(K, 2, 2);
+  const S w0 = v[0], w1 = v[1], w2 = v[2];
+  B[0] = fma_s(S(xz), w1, S(-xy) * w2);
+  B[3] = fma_s(S(xy), w2, S(-yz) * w0);
+  B[5] = fma_s(S(yz), w0, S(-xz) * w1);
+  B[1] = fma_s(S(0.5 * (xx - yy)), w2, fma_s(S(0.5 * yz), w1, S(-0.5 * xz) * w0));
+  B[2] = fma_s(S(0.5 * (zz - xx)), w1, fma_s(S(-0.5 * yz), w2, S(0.5 * xy) * w0));
+  B[4] = fma_s(S(0.5 * (yy - zz)), w0, fma_s(S(0.5 * xz), w2, S(-0.5 * xy) * w1));
+  add_sym_outer<S>(S(0.5), S(first_moment<K>(0)), S(first_moment<K>(1)), S(first_moment<K>(2)), v + 3, B);
+}
+
+// D = 2 v x S (entries 2 and 5 are zero) and P = a x S + v x (v x S)
+template <typename S>
+RBD_HD RBD_INLINE void motion_pair(const S* v, const S* a, S D[6], S P[6]) {
+  D[0] = v[1] + v[1]; D[1] = -(v[0] + v[0]); D[2] = S(0);
+  D[3] = v[4] + v[4]; D[4] = -(v[3] + v[3]); D[5] = S(0);
+  P[0] = fma_s(v[2], v[0], a[1]);
+  P[1] = fma_s(v[2], v[1], -a[0]);
+  P[2] = fma_s(-v[0], v[0], -(v[1] * v[1]));
+  P[3] = fma_s(v[2], v[3], fma_s(v[5], v[0], a[4]));
+  P[4] = fma_s(v[2], v[4], fma_s(v[5], v[1], -a[3]));
+  P[5] = fma_s(D[1], v[3], -(D[0] * v[4]));
+}
+
+// What a column needs of each link besides its transform: Bs, P and D.  In FP32
+// they are stored (a lane of a group runs up to four columns); in FP64, where
+// they would take 280 registers more and the kernels spill, they are formed
+// again from v and a in each column.
+template <typename S, bool STORED = sizeof(S) == 4>
+struct LinkTerms {
+  S b[NQ][6], P[NQ][6], D[NQ][6];
+  template <int K> RBD_HD RBD_INLINE void set(const S* v, const S* a) {
+    body_bs<K>(v, b[K]);
+    motion_pair(v, a, D[K], P[K]);
+  }
+  template <int K> RBD_HD RBD_INLINE void get(S bk[6], S Dk[6], S Pk[6]) const {
+    for (int i = 0; i < 6; ++i) { bk[i] = b[K][i]; Dk[i] = D[K][i]; Pk[i] = P[K][i]; }
+  }
+  RBD_HD RBD_INLINE void forget() {}
+};
+template <typename S>
+struct LinkTerms<S, false> {
+  S v[NQ][6], a[NQ][6];
+  template <int K> RBD_HD RBD_INLINE void set(const S* vk, const S* ak) {
+    for (int i = 0; i < 6; ++i) { v[K][i] = vk[i]; a[K][i] = ak[i]; }
+  }
+  template <int K> RBD_HD RBD_INLINE void get(S bk[6], S Dk[6], S Pk[6]) const {
+    body_bs<K>(v[K], bk);
+    motion_pair(v[K], a[K], Dk, Pk);
+  }
+  // between two columns of a lane: keeps the compiler from holding the first
+  // column's terms for the second
+  RBD_HD RBD_INLINE void forget() {
+#if defined(__HIP_DEVICE_COMPILE__)
+    for (int k = 0; k < NQ; ++k)
+      for (int i = 0; i < 6; ++i) asm volatile("" : "+v"(v[k][i]));
+#endif
+  }
+};
+
 template <typename S>
 struct PhaseC {
   CS<S> t[NQ];
-  S v[NQ][6];      // link velocities
-  S Iv[NQ][6];     // I_k v_k
-  S axs[NQ][4];    // a_k x S  -> (a1, -a0, a4, -a3)   (entries 2 and 5 are zero)
+  LinkTerms<S> link;
+  S n[NQ][3], p[NQ][3];   // momentum of each link
   S nfxs[NQ][4];   // -(f_k x S) -> (-f1, f0, -f4, f3)
-  S qd[NQ];
   S Mi[NQ][NQ];    // upper triangle of Minv
 };
-
-// dtau[:, c] for the d/dqd (DQ == false) or d/dq (DQ == true) column c.
-template <bool DQ, typename S>
-RBD_HD RBD_INLINE void dtau_column(const PhaseC<S>& P, int c, S tau[NQ]) {
-  S dv[6], da[6], df[NQ][6];
-  static_for<0, NQ>([&](auto Kc) {
-    constexpr int k = decltype(Kc)::value;
-    if (k < c) {
-      for (int i = 0; i < 6; ++i) df[k][i] = S(0);
-      return;
-    }
-    if (k == c) {
-      if constexpr (DQ) {
-        dv[0] = P.v[k][1]; dv[1] = -P.v[k][0]; dv[2] = S(0);
-        dv[3] = P.v[k][4]; dv[4] = -P.v[k][3]; dv[5] = S(0);
-        da[0] = P.axs[k][0]; da[1] = P.axs[k][1]; da[2] = S(0);
-        da[3] = P.axs[k][2]; da[4] = P.axs[k][3]; da[5] = S(0);
-      } else {
-        for (int i = 0; i < 6; ++i) dv[i] = S(0);
-        dv[2] = S(1);
-        da[0] = P.v[k][1]; da[1] = -P.v[k][0]; da[2] = S(0);
-        da[3] = P.v[k][4]; da[4] = -P.v[k][3]; da[5] = S(0);
-      }
-    } else {
-      if constexpr (k > 0) {
-        S y[6];
-        xmotion<k>(P.t[k], dv, y);
-        for (int i = 0; i < 6; ++i) dv[i] = y[i];
-        xmotion<k>(P.t[k], da, y);
-        const S qk = P.qd[k];
-        da[0] = y[0] + dv[1] * qk; da[1] = y[1] - dv[0] * qk; da[2] = y[2];
-        da[3] = y[3] + dv[4] * qk; da[4] = y[4] - dv[3] * qk; da[5] = y[5];
-      }
-    }
-    S Idv[6];
-    imv<k>(dv, Idv);
-    imv<k>(da, df[k]);
-    crf<true>(dv, P.Iv[k], df[k]);
-    crf<true>(P.v[k], Idv, df[k]);
-  });
-  S g[6];
-  for (int i = 0; i < 6; ++i) g[i] = df[NQ - 1][i];
-  static_for_down<NQ, 1>([&](auto Kc) {
-    constexpr int k = decltype(Kc)::value;
-    tau[k] = g[2];
-    if constexpr (DQ) {
-      if (k == c) {
-        g[0] += P.nfxs[k][0]; g[1] += P.nfxs[k][1];
-        g[3] += P.nfxs[k][2]; g[4] += P.nfxs[k][3];
-      }
-    }
-    S y[6];
-    if (k - 1 >= c) xforce_t_add<k>(P.t[k], g, df[k - 1], y);
-    else            xforce_t<k>(P.t[k], g, y);
-    for (int i = 0; i < 6; ++i) g[i] = y[i];
-  });
-  tau[0] = g[2];
-}
 
 // tau[c] += x for a run-time c without indexing a register array
 template <typename S>
@@ -620,41 +802,38 @@ RBD_HD RBD_INLINE void minv_times(const S Mi[NQ][NQ], const SX x[NQ], SX out[NQ]
   });
 }
 
-// Uniform-sweep variant of dtau_column for lane-parallel use: the column c and
-// its kind (dq) may differ from lane to lane while every lane executes the same
-// instructions.  dv, da start at zero and stay zero until k == c, where the seed
-// replaces them by select; the zero df_k for k < c then adds exactly nothing in
-// the backward sweep, so the result equals dtau_column's.
+// dtau of one derivative column for lane-parallel use: the column c and its
+// kind (dq) may differ from lane to lane while every lane executes the same
+// instructions.  The moved vectors x (6) and w (the angular part that B sees)
+// start at zero and stay zero until k == c, where the seed replaces them by
+// select; the zero df_k for k < c then adds exactly nothing in the backward
+// sweep.
 template <typename S>
 RBD_HD RBD_INLINE void dtau_column_uniform(const PhaseC<S>& P, int c, bool dq, S tau[NQ]) {
-  S dv[6], da[6], df[NQ][6];
-  for (int i = 0; i < 6; ++i) { dv[i] = S(0); da[i] = S(0); }
+  S x[6], w[3], df[NQ][6];
+  for (int i = 0; i < 6; ++i) x[i] = S(0);
+  for (int i = 0; i < 3; ++i) w[i] = S(0);
   static_for<0, NQ>([&](auto Kc) {
     constexpr int k = decltype(Kc)::value;
-    S pv[6], pa[6];
     if constexpr (k > 0) {
-      xmotion<k>(P.t[k], dv, pv);
-      xmotion<k>(P.t[k], da, pa);
-      const S qk = P.qd[k];
-      pa[0] += pv[1] * qk; pa[1] -= pv[0] * qk; pa[3] += pv[4] * qk; pa[4] -= pv[3] * qk;
-    } else {
-      for (int i = 0; i < 6; ++i) { pv[i] = S(0); pa[i] = S(0); }
+      move_motion<k>(P.t[k], x, x);
+      to_child<k>(P.t[k], w, w);
     }
-    // seeds: d/dqd -> dv = S, da = v_k x S;  d/dq -> dv = v_k x S, da = a_k x S
-    const S vx[6] = {P.v[k][1], -P.v[k][0], S(0), P.v[k][4], -P.v[k][3], S(0)};
-    const S ax[6] = {P.axs[k][0], P.axs[k][1], S(0), P.axs[k][2], P.axs[k][3], S(0)};
+    S b[6], Dk[6], Pk[6];
+    P.link.template get<k>(b, Dk, Pk);
     const bool seed = (k == c);
-    for (int i = 0; i < 6; ++i) {
-      const S sv = dq ? vx[i] : (i == 2 ? S(1) : S(0));
-      const S sa = dq ? ax[i] : vx[i];
-      dv[i] = seed ? sv : pv[i];
-      da[i] = seed ? sa : pa[i];
-    }
-    S Idv[6];
-    imv<k>(dv, Idv);
-    imv<k>(da, df[k]);
-    crf<true>(dv, P.Iv[k], df[k]);
-    crf<true>(P.v[k], Idv, df[k]);
+    for (int i = 0; i < 6; ++i) x[i] = seed ? (dq ? Pk[i] : Dk[i]) : x[i];
+    for (int i = 0; i < 3; ++i) w[i] = seed ? (dq ? Dk[i] : (i == 2 ? S(2) : S(0))) : w[i];
+    inertia_times<k>(x, df[k]);
+    const S* n = P.n[k]; const S* p = P.p[k];
+    // += [(Bs - n^ / 2) w; -p x w], n^ w / 2 = n x w / 2
+    const S h[3] = {S(0.5) * w[0], S(0.5) * w[1], S(0.5) * w[2]};
+    df[k][0] = fma_s(b[0], w[0], fma_s(b[1], w[1], fma_s(b[2], w[2], fma_s(n[2], h[1], fma_s(-n[1], h[2], df[k][0])))));
+    df[k][1] = fma_s(b[1], w[0], fma_s(b[3], w[1], fma_s(b[4], w[2], fma_s(n[0], h[2], fma_s(-n[2], h[0], df[k][1])))));
+    df[k][2] = fma_s(b[2], w[0], fma_s(b[4], w[1], fma_s(b[5], w[2], fma_s(n[1], h[0], fma_s(-n[0], h[1], df[k][2])))));
+    df[k][3] = fma_s(p[2], w[1], fma_s(-p[1], w[2], df[k][3]));
+    df[k][4] = fma_s(p[0], w[2], fma_s(-p[2], w[0], df[k][4]));
+    df[k][5] = fma_s(p[1], w[0], fma_s(-p[0], w[1], df[k][5]));
   });
   S g[6];
   for (int i = 0; i < 6; ++i) g[i] = df[NQ - 1][i];
@@ -664,68 +843,287 @@ RBD_HD RBD_INLINE void dtau_column_uniform(const PhaseC<S>& P, int c, bool dq, S
     const bool extra = dq && (k == c);
     g[0] += extra ? P.nfxs[k][0] : S(0); g[1] += extra ? P.nfxs[k][1] : S(0);
     g[3] += extra ? P.nfxs[k][2] : S(0); g[4] += extra ? P.nfxs[k][3] : S(0);
-    S y[6];
-    xforce_t_add<k>(P.t[k], g, df[k - 1], y);
-    for (int i = 0; i < 6; ++i) g[i] = y[i];
+    add_moved_force<k>(P.t[k], g, df[k - 1]);
+    for (int i = 0; i < 6; ++i) g[i] = df[k - 1][i];
   });
   tau[0] = g[2];
 }
 
 // Phase-C inputs from v, a (with qdd), f (after the backward pass) and Minv.
 template <typename SC, typename SR, typename SM>
-RBD_HD RBD_INLINE void make_phase_c(PhaseC<SC>& P, const CS<SC>* t, const SR* qd, const SR v[NQ][6],
-                                    const SR a[NQ][6], const SR f[NQ][6], const SM Mi[NQ][NQ]) {
-  for (int k = 0; k < NQ; ++k) { P.t[k] = t[k]; P.qd[k] = SC(qd[k]); }
+RBD_HD RBD_INLINE void make_phase_c(PhaseC<SC>& P, const CS<SC>* t, const SR v[NQ][6], const SR a[NQ][6],
+                                    const SR f[NQ][6], const SM Mi[NQ][NQ]) {
+  for (int k = 0; k < NQ; ++k) P.t[k] = t[k];
   for (int r = 0; r < NQ; ++r)
     for (int c = r; c < NQ; ++c) P.Mi[r][c] = SC(Mi[r][c]);
   static_for<0, NQ>([&](auto Kc) {
     constexpr int k = decltype(Kc)::value;
-    for (int i = 0; i < 6; ++i) P.v[k][i] = SC(v[k][i]);
-    imv<k>(P.v[k], P.Iv[k]);
-    P.axs[k][0] = SC(a[k][1]); P.axs[k][1] = -SC(a[k][0]); P.axs[k][2] = SC(a[k][4]); P.axs[k][3] = -SC(a[k][3]);
+    SC vk[6], ak[6], h[6];
+    for (int i = 0; i < 6; ++i) { vk[i] = SC(v[k][i]); ak[i] = SC(a[k][i]); }
+    inertia_times<k>(vk, h);
+    for (int i = 0; i < 3; ++i) { P.n[k][i] = h[i]; P.p[k][i] = h[3 + i]; }
+    P.link.template set<k>(vk, ak);
     P.nfxs[k][0] = -SC(f[k][1]); P.nfxs[k][1] = SC(f[k][0]); P.nfxs[k][2] = -SC(f[k][4]); P.nfxs[k][3] = SC(f[k][3]);
   });
 }
 
-// The d/dq columns in one lane (one lane per knot) and their stores.  MINV =
-// false stores the inverse-dynamics gradient dtau/dq itself (the reference's
-// cdu) instead of -Minv times it.
-template <bool MINV = true, typename SC, class Out>
-RBD_HD RBD_INLINE void gradient_dq_columns(const PhaseC<SC>& P, Out& out) {
-  // d/dq column 0 is identically zero (rotation about the gravity axis)
-  for (int r = 0; r < NQ; ++r) out.dq(r, 0, 0.0f);
-  static_for<1, NQ>([&](auto Cc) {
-    constexpr int c = decltype(Cc)::value;
-    SC tau[NQ], col[NQ];
-    dtau_column<true>(P, c, tau);
-    if constexpr (MINV) minv_times<true>(P.Mi, tau, col);
-    else for (int r = 0; r < NQ; ++r) col[r] = tau[r];
-    for (int r = 0; r < NQ; ++r) out.dq(r, c, float(col[r]));
+// ---------------------------------------------------------------------------
+// All derivative columns in one lane, from composite quantities.
+//
+// In df_k above only I_k and B_k depend on the link, so the backward sweep's
+// sum over the links from c on is a product with their composite inertia IC_c
+// and composite B_c.  Both composites are a few numbers: IC six and three
+// (its mass is a constant), B six and the composite momentum.  Going from the
+// tip to the base, link c gives
+//   rows j <= c of column c:  S_j . (IC P + B D + S x* f) and S_j . (IC D + 2 B S),
+//   columns j < c of row c:   (IC S) . P_j + (B^T S) . D_j and (IC S) . D_j + 2 (B^T S) . S_j
+// where the four force vectors (the last a pure couple) are moved down the
+// links j < c.  That is 21 moves of three and a half vectors in place of the
+// thirteen columns' sweeps over up to seven links forward and back (2,300
+// instructions against 3,700; Singh, Russell and Wensing, "Efficient
+// analytical derivatives of rigid-body dynamics using spatial vector
+// algebra", 2022, give the world-frame form).
+// ---------------------------------------------------------------------------
+// mass of the links from K on
+template <int K>
+RBD_HD constexpr double composite_mass() {
+  double m = 0.0;
+  for (int j = K; j < NQ; ++j) m += inertia_entry(j, 3, 3);
+  return m;
+}
+template <typename S> struct Composite {
+  S i[6], h[3];    // composite inertia: about the link's origin, first moment
+  S b[6];          // Bs
+  S n[3], p[3];    // momentum
+  S f[6];          // force on the link from the links from here on
+};
+
+// Link K joins the composite, which moves from link K + 1's frame to its own.
+// f_given: the force on the link (the reference's split layout) instead of
+// the composite's own sum.
+template <int K, bool F_GIVEN, class In, typename S>
+RBD_HD RBD_INLINE void composite_step(const In& in, const CS<S>* t, const S* v, const S* a, Composite<S>& c) {
+  S h[6], B[6];
+  inertia_times<K>(v, h);
+  body_bs<K>(v, B);
+  S f[6];
+  if constexpr (F_GIVEN) {
+    for (int i = 0; i < 6; ++i) f[i] = S(in.f(K, i));
+  } else {
+    inertia_times<K>(a, f);
+    add_force_cross(v, h, f);
+    if (in.fx)
+      for (int i = 0; i < 6; ++i) f[i] -= S(in.fx[6 * K + i]);
+  }
+  if constexpr (K == NQ - 1) {
+    static_for<0, 3>([&](auto Ic) {
+      constexpr int i = decltype(Ic)::value;
+      static_for<i, 3>([&](auto Jc) {
+        constexpr int j = decltype(Jc)::value;
+        c.i[sym(i, j)] = kInertia<S, K, i, j>;
+      });
+      c.h[i] = S(first_moment<K>(i));
+      c.n[i] = h[i];
+      c.p[i] = h[3 + i];
+    });
+    for (int i = 0; i < 6; ++i) { c.b[i] = B[i]; c.f[i] = f[i]; }
+  } else {
+    constexpr int u = K + 1;
+    constexpr double r[3] = {kJointOffset[u][0], kJointOffset[u][1], kJointOffset[u][2]};
+    constexpr double m = composite_mass<u>();
+    constexpr double rr = r[0] * r[0] + r[1] * r[1] + r[2] * r[2];
+    const DoubleAngle<S> q = double_angle(t[u]);
+    // inertia about the new origin: i + 2 (r.h) 1 - h r^T - r h^T + m (r.r 1 - r r^T), then the link's own
+    to_parent<u>(t[u], c.h, c.h);
+    sym_to_parent<u>(t[u], q, c.i);
+    add_sym_outer<S>(S(1), S(r[0]), S(r[1]), S(r[2]), c.h, c.i);
+    static_for<0, 3>([&](auto Ic) {
+      constexpr int i = decltype(Ic)::value;
+      constexpr double hk = m * r[i] + first_moment<K>(i);
+      c.h[i] += S(hk);
+      static_for<i, 3>([&](auto Jc) {
+        constexpr int j = decltype(Jc)::value;
+        constexpr double ik = inertia_entry(K, i, j) + m * ((i == j ? rr : 0.0) - r[i] * r[j]);
+        c.i[sym(i, j)] += S(ik);
+      });
+    });
+    // Bs likewise with the momentum p in h's place; the momentum moves as a force
+    to_parent<u>(t[u], c.p, c.p);
+    sym_to_parent<u>(t[u], q, c.b);
+    add_sym_outer<S>(S(0.5), S(r[0]), S(r[1]), S(r[2]), c.p, c.b);
+    for (int i = 0; i < 6; ++i) c.b[i] += B[i];
+    to_parent_add<u>(t[u], c.n, h, c.n);
+    add_offset_cross<u>(c.p, c.n);
+    for (int i = 0; i < 3; ++i) c.p[i] += h[3 + i];
+    if constexpr (!F_GIVEN) add_moved_force<u>(t[u], c.f, f);
+    for (int i = 0; i < 6; ++i) c.f[i] = f[i];
+  }
+}
+
+// The columns from the tip's to the base's: emit(IC<c>, dtau/dq_c, dtau/dqd_c)
+// (the d/dq column 0 is identically zero: rotation about the gravity axis).
+template <bool F_GIVEN = false, class In, typename S, class Emit>
+RBD_HD RBD_INLINE void derivative_columns(const In& in, const CS<S>* t, const S v[NQ][6], const S a[NQ][6],
+                                          Emit&& emit) {
+  S tq[NQ][NQ], td[NQ][NQ];        // dtau/dq, dtau/dqd: [row][column]
+  Composite<S> c;
+  static_for_down<NQ, 0>([&](auto Kc) {
+    constexpr int k = decltype(Kc)::value;
+    constexpr S m = S(composite_mass<k>());
+    composite_step<k, F_GIVEN>(in, t, v[k], a[k], c);
+    const S b01 = fma_s(S(0.5), c.n[2], c.b[1]), b10 = fma_s(S(-0.5), c.n[2], c.b[1]);
+    const S b02 = fma_s(S(-0.5), c.n[1], c.b[2]), b20 = fma_s(S(0.5), c.n[1], c.b[2]);
+    const S b12 = fma_s(S(0.5), c.n[0], c.b[4]), b21 = fma_s(S(-0.5), c.n[0], c.b[4]);
+    S D[6], P[6];
+    motion_pair(v[k], a[k], D, P);
+    S is[6] = {c.i[2], c.i[4], c.i[5], -c.h[1], c.h[0], S(0)};       // IC S
+    S bs[3] = {b20, b21, c.b[5]};                                    // B^T S
+    S g[6], gd[6];                                                    // IC P + B D + S x* f, IC D + 2 B S
+    gd[0] = fma_s(c.i[0], D[0], fma_s(c.i[1], D[1], fma_s(-c.h[2], D[4], S(2) * b02)));
+    gd[1] = fma_s(c.i[1], D[0], fma_s(c.i[3], D[1], fma_s(c.h[2], D[3], S(2) * b12)));
+    gd[2] = fma_s(c.i[2], D[0], fma_s(c.i[4], D[1], fma_s(c.h[0], D[4], fma_s(-c.h[1], D[3], S(2) * c.b[5]))));
+    gd[3] = fma_s(m, D[3], fma_s(c.h[2], D[1], S(-2) * c.p[1]));
+    gd[4] = fma_s(m, D[4], fma_s(-c.h[2], D[0], S(2) * c.p[0]));
+    gd[5] = fma_s(c.h[1], D[0], -(c.h[0] * D[1]));
+    td[k][k] = gd[2];
+    if constexpr (k > 0) {
+      g[0] = fma_s(c.i[0], P[0], fma_s(c.i[1], P[1], fma_s(c.i[2], P[2], fma_s(c.h[1], P[5], fma_s(-c.h[2], P[4],
+             fma_s(c.b[0], D[0], fma_s(b01, D[1], -c.f[1])))))));
+      g[1] = fma_s(c.i[1], P[0], fma_s(c.i[3], P[1], fma_s(c.i[4], P[2], fma_s(c.h[2], P[3], fma_s(-c.h[0], P[5],
+             fma_s(b10, D[0], fma_s(c.b[3], D[1], c.f[0])))))));
+      g[2] = fma_s(c.i[2], P[0], fma_s(c.i[4], P[1], fma_s(c.i[5], P[2], fma_s(c.h[0], P[4], fma_s(-c.h[1], P[3],
+             fma_s(b20, D[0], b21 * D[1]))))));
+      g[3] = fma_s(m, P[3], fma_s(c.h[2], P[1], fma_s(-c.h[1], P[2], fma_s(c.p[2], D[1], -c.f[4]))));
+      g[4] = fma_s(m, P[4], fma_s(c.h[0], P[2], fma_s(-c.h[2], P[0], fma_s(-c.p[2], D[0], c.f[3]))));
+      g[5] = fma_s(m, P[5], fma_s(c.h[1], P[0], fma_s(-c.h[0], P[1], fma_s(c.p[1], D[0], -(c.p[0] * D[1])))));
+      tq[k][k] = g[2];
+      static_for_down<k + 1, 1>([&](auto Uc) {
+        constexpr int u = decltype(Uc)::value, j = u - 1;             // from link u to link j
+        move_force<u>(t[u], g);
+        move_force<u>(t[u], gd);
+        move_force<u>(t[u], is);
+        to_parent<u>(t[u], bs, bs);
+        tq[j][k] = g[2];
+        td[j][k] = gd[2];
+        if constexpr (j > 0) {
+          S Dj[6], Pj[6];
+          motion_pair(v[j], a[j], Dj, Pj);
+          td[k][j] = fma_s(is[0], Dj[0], fma_s(is[1], Dj[1], fma_s(is[3], Dj[3], fma_s(is[4], Dj[4], S(2) * bs[2]))));
+          tq[k][j] = fma_s(is[0], Pj[0], fma_s(is[1], Pj[1], fma_s(is[2], Pj[2], fma_s(is[3], Pj[3],
+                     fma_s(is[4], Pj[4], fma_s(is[5], Pj[5], fma_s(bs[0], Dj[0], bs[1] * Dj[1])))))));
+        } else {
+          td[k][0] = S(2) * bs[2];                                     // link 0 only turns: D_0 = 0
+        }
+      });
+    }
+    S cq[NQ], cd[NQ];
+    static_for<0, NQ>([&](auto Rc) {
+      constexpr int r = decltype(Rc)::value;
+      if constexpr (k > 0) cq[r] = tq[r][k];
+      else cq[r] = S(0);
+      cd[r] = td[r][k];
+    });
+    emit(Kc, cq, cd);
   });
 }
 
-// The d/dqd columns in one lane and their stores (damping on the diagonal).
-template <bool MINV = true, typename SC, class Out>
-RBD_HD RBD_INLINE void gradient_dqd_columns(const PhaseC<SC>& P, float damping, Out& out) {
-  static_for<0, NQ>([&](auto Cc) {
-    constexpr int c = decltype(Cc)::value;
-    SC tau[NQ], col[NQ];
-    dtau_column<false>(P, c, tau);
-    add_on_diagonal(tau, c, SC(damping));
-    if constexpr (MINV) minv_times<true>(P.Mi, tau, col);
-    else for (int r = 0; r < NQ; ++r) col[r] = tau[r];
-    for (int r = 0; r < NQ; ++r) out.dqd(r, c, float(col[r]));
+// Link velocities and accelerations in one lane (RNEA_fp's recursions,
+// dynamicsGradient.h:619-659); qdd null: zero joint accelerations.
+template <typename S>
+RBD_HD RBD_INLINE void link_motion(const CS<S>* t, const S* qd, const S* qdd, S gravity, S v[NQ][6], S a[NQ][6]) {
+  static_for<0, NQ>([&](auto Kc) {
+    constexpr int k = decltype(Kc)::value;
+    if constexpr (k == 0) {
+      for (int i = 0; i < 6; ++i) { v[0][i] = S(0); a[0][i] = S(0); }
+      v[0][2] = qd[0];
+      const S g[3] = {S(0), S(0), gravity};
+      to_child<0>(t[0], g, a[0] + 3);              // T_0 [0,0,0,0,0,g] = [0; E g]
+    } else {
+      move_motion<k>(t[k], v[k - 1], v[k]);
+      v[k][2] += qd[k];
+      move_motion<k>(t[k], a[k - 1], a[k]);
+      a[k][0] = fma_s(v[k][1], qd[k], a[k][0]);    // + (v x S) qd
+      a[k][1] = fma_s(-v[k][0], qd[k], a[k][1]);
+      a[k][3] = fma_s(v[k][4], qd[k], a[k][3]);
+      a[k][4] = fma_s(-v[k][3], qd[k], a[k][4]);
+    }
+    if (qdd) a[k][2] += qdd[k];
+  });
+}
+// a += the accelerations that qdd adds
+template <typename S>
+RBD_HD RBD_INLINE void add_joint_accelerations(const CS<S>* t, const S* qdd, S a[NQ][6]) {
+  S d[6] = {S(0), S(0), qdd[0], S(0), S(0), S(0)};
+  a[0][2] += qdd[0];
+  static_for<1, NQ>([&](auto Kc) {
+    constexpr int k = decltype(Kc)::value;
+    move_motion<k>(t[k], d, d);
+    d[2] += qdd[k];
+    for (int i = 0; i < 6; ++i) a[k][i] += d[i];
+  });
+}
+// Link forces and joint torques of a motion, from the tip (RNEA_bp,
+// dynamicsGradient.h:661-670): sink(IC<k>, the force on link k), its entry 2 the torque
+template <class In, typename S, class Sink>
+RBD_HD RBD_INLINE void link_forces(const In& in, const CS<S>* t, const S v[NQ][6], const S a[NQ][6], Sink&& sink) {
+  S f[6];
+  static_for_down<NQ, 0>([&](auto Kc) {
+    constexpr int k = decltype(Kc)::value;
+    S h[6], b[6];
+    inertia_times<k>(v[k], h);
+    inertia_times<k>(a[k], b);
+    add_force_cross(v[k], h, b);
+    if (in.fx)
+      for (int i = 0; i < 6; ++i) b[i] -= S(in.fx[6 * k + i]);
+    if constexpr (k < NQ - 1) add_moved_force<k + 1>(t[k + 1], f, b);
+    for (int i = 0; i < 6; ++i) f[i] = b[i];
+    sink(Kc, f);
   });
 }
 
-// All derivative columns in one lane and the stores of dqdd/dq, dqdd/dqd: the
-// d/dq columns, then the d/dqd columns -- the order of the outputs in memory,
-// so that each knot's AoS record fills front to back and few of its cache
-// lines are partly written at a time.
-template <bool MINV = true, typename SC, class Out>
-RBD_HD RBD_INLINE void gradient_columns(const PhaseC<SC>& P, float damping, Out& out) {
-  gradient_dq_columns<MINV>(P, out);
-  gradient_dqd_columns<MINV>(P, damping, out);
+// The columns' last step and their stores: times -Minv through the factors of
+// M, times a given -Minv (upper triangle), or none (the inverse-dynamics
+// gradient itself, the reference's cdu).
+template <typename S> struct TimesMassInverse {
+  const MassFactors<S>& f;
+  template <typename SX> RBD_HD RBD_INLINE void operator()(SX x[NQ]) const { mass_solve<true>(f, x); }
+};
+template <typename S> struct TimesMinv {
+  const S (*Mi)[NQ];
+  template <typename SX> RBD_HD RBD_INLINE void operator()(SX x[NQ]) const {
+    SX y[NQ];
+    static_for<0, NQ>([&](auto Rc) {
+      constexpr int r = decltype(Rc)::value;
+      SX acc = -SX(Mi[0][r]) * x[0];
+      static_for<1, NQ>([&](auto Cc) {
+        constexpr int c = decltype(Cc)::value;
+        acc = fma_s(-SX(r <= c ? Mi[r][c] : Mi[c][r]), x[c], acc);
+      });
+      y[r] = acc;
+    });
+    for (int r = 0; r < NQ; ++r) x[r] = y[r];
+  }
+};
+struct TimesNothing {
+  template <typename SX> RBD_HD RBD_INLINE void operator()(SX*) const {}
+};
+template <bool F_GIVEN = false, class In, typename S, class Times, class Out>
+RBD_HD RBD_INLINE void gradient_columns(const In& in, const CS<S>* t, const S v[NQ][6], const S a[NQ][6],
+                                        float damping, const Times& times, Out& out) {
+  derivative_columns<F_GIVEN>(in, t, v, a, [&](auto Cc, S* cq, S* cd) {
+    constexpr int c = decltype(Cc)::value;
+    cd[c] += S(damping);
+    times(cd);
+    if constexpr (c > 0) times(cq);
+    static_for<0, NQ>([&](auto Rc) {
+      constexpr int r = decltype(Rc)::value;
+      out.dq(r, c, float(cq[r]));
+    });
+    static_for<0, NQ>([&](auto Rc) {
+      constexpr int r = decltype(Rc)::value;
+      out.dqd(r, c, float(cd[r]));
+    });
+  });
 }
 
 // Lane roles when one knot is spread over a group of kLanesPerKnotGroup lanes:
@@ -791,15 +1189,17 @@ RBD_HD RBD_INLINE bool bounded_wait(Poll&& poll, Pause&& pause, int spins) {
 template <class P>
 using KnotTrig = Wider<typename P::Minv, Wider<typename P::Rnea, typename P::Col>>;
 
-template <class P, class In>
-RBD_HD RBD_INLINE void knot_trig(const In& in, CS<KnotTrig<P>> tw[NQ]) {
-  using ST = KnotTrig<P>;
+// sin/cos of a knot's joints in one lane, in type ST
+template <class P, typename ST, class In>
+RBD_HD RBD_INLINE void knot_trig_in(P, const In& in, CS<ST> tw[NQ]) {
   for (int k = 0; k < NQ; ++k) {
     ST s, c;
     knot_sincos<P>(ST(in.q(k)), &s, &c);
     tw[k] = CS<ST>{c, s};
   }
 }
+template <class P, class In>
+RBD_HD RBD_INLINE void knot_trig(const In& in, CS<KnotTrig<P>> tw[NQ]) { knot_trig_in(P{}, in, tw); }
 
 // The same for a knot's lane group: lane role j < 7 computes the sin/cos of
 // q_j alone and the group's lanes read all seven from each other by
@@ -861,22 +1261,7 @@ RBD_HD RBD_INLINE void phase_a_after_minv(const In& in, const Options& opt, cons
     for (int k = 0; k < NQ; ++k)
       for (int i = 0; i < 6; ++i) f[k][i] += dF[k][i];
   }
-  make_phase_c(PC, tc, qd, v, a, f, Mi);
-}
-
-// Steps 1-5 of the full path: sin/cos, Minv, bias RNEA, qdd = Minv (u - c), RNEA
-// with qdd; fills the phase-C inputs and qdd.
-template <class P, class In>
-RBD_HD RBD_INLINE void phase_a(const In& in, const Options& opt, PhaseC<typename P::Col>& PC,
-                               typename P::Rnea qdd[NQ]) {
-  using SM = typename P::Minv; using SP = typename P::Pivot;
-  CS<KnotTrig<P>> tw[NQ];
-  knot_trig<P>(in, tw);
-  CS<SM> tm[NQ];
-  for (int k = 0; k < NQ; ++k) tm[k] = CS<SM>{SM(tw[k].c), SM(tw[k].s)};
-  SM Mi[NQ][NQ];
-  compute_minv<SM, SP>(tm, Mi);
-  phase_a_after_minv<P>(in, opt, tw, Mi, PC, qdd);
+  make_phase_c(PC, tc, v, a, f, Mi);
 }
 
 // Steps 1 and 5 of the reference-compatible modes: qdd given, and with
@@ -887,10 +1272,10 @@ RBD_HD RBD_INLINE void phase_a_given_qdd_minv(const In& in, const Options& opt, 
   using ST = Wider<SR, SC>;
   CS<SR> tr[NQ]; CS<SC> tc[NQ];
   SR qd[NQ], qdd[NQ];
+  CS<ST> tw[NQ];
+  knot_trig_in(P{}, in, tw);
   for (int k = 0; k < NQ; ++k) {
-    ST s, c;
-    knot_sincos<P>(ST(in.q(k)), &s, &c);
-    tr[k] = CS<SR>{SR(c), SR(s)}; tc[k] = CS<SC>{SC(c), SC(s)};
+    tr[k] = CS<SR>{SR(tw[k].c), SR(tw[k].s)}; tc[k] = CS<SC>{SC(tw[k].c), SC(tw[k].s)};
     qd[k] = SR(in.qd(k));
     qdd[k] = SR(in.qdd(k));
   }
@@ -904,12 +1289,19 @@ RBD_HD RBD_INLINE void phase_a_given_qdd_minv(const In& in, const Options& opt, 
   rnea_fwd(tr, qd, qdd, SR(opt.gravity), v, a, f);
   subtract_fext(in, f);
   rnea_bwd(tr, f);
-  make_phase_c(PC, tc, qd, v, a, f, Mi);
+  make_phase_c(PC, tc, v, a, f, Mi);
 }
 
 // Output accessors that also want dqdd/du = Minv (dense) declare kMinv = true.
 template <class Out, class = void> struct WantsMinv { static constexpr bool value = false; };
 template <class Out> struct WantsMinv<Out, typename std::enable_if<Out::kMinv>::type> {
+  static constexpr bool value = true;
+};
+
+// Those that want to know when Minv is complete, before anything else is
+// stored, have a minv_done().
+template <class Out, class = void> struct StagesMinv { static constexpr bool value = false; };
+template <class Out> struct StagesMinv<Out, decltype(static_cast<const Out*>(nullptr)->minv_done())> {
   static constexpr bool value = true;
 };
 
@@ -927,17 +1319,75 @@ RBD_HD RBD_INLINE void store_minv_column(Out& out, const S Mi[NQ][NQ], int c) {
   });
 }
 
+// sin/cos in the type S of a phase
+template <typename S, typename ST>
+RBD_HD RBD_INLINE void cast_trig(const CS<ST> tw[NQ], CS<S> t[NQ]) {
+  for (int k = 0; k < NQ; ++k) t[k] = CS<S>{S(tw[k].c), S(tw[k].s)};
+}
+
+// Steps 1-4 of the full path in one lane: sin/cos, the factors of M, bias RNEA,
+// qdd = M^-1 (u - c); v and a (the latter at qdd = 0) for the gradient.
+template <class P, class In>
+RBD_HD RBD_INLINE void knot_forward_dynamics(const In& in, const Options& opt, const CS<KnotTrig<P>> tw[NQ],
+                                             MassFactors<typename P::Minv>& f, typename P::Rnea v[NQ][6],
+                                             typename P::Rnea a[NQ][6], typename P::Rnea qdd[NQ]) {
+  using SM = typename P::Minv; using SP = typename P::Pivot; using SR = typename P::Rnea;
+  CS<SM> tm[NQ]; CS<SR> tr[NQ];
+  cast_trig(tw, tm);
+  cast_trig(tw, tr);
+  mass_factors<SM, SP>(tm, f);
+  SR qd[NQ];
+  for (int k = 0; k < NQ; ++k) qd[k] = SR(in.qd(k));
+  link_motion(tr, qd, static_cast<const SR*>(nullptr), SR(opt.gravity), v, a);
+  link_forces(in, tr, v, a, [&](auto Kc, const SR* fk) {
+    constexpr int k = decltype(Kc)::value;
+    qdd[k] = fma_s(-SR(opt.damping), qd[k], SR(in.u(k)) - fk[2]);
+  });
+  mass_solve<false>(f, qdd);
+}
+
+// Minv (dense) to out.minv
+template <class Out, typename S>
+RBD_HD RBD_INLINE void store_minv(Out& out, const MassFactors<S>& f) {
+  S Mi[NQ][NQ];
+  minv_from_factors(f, Mi);
+  static_for<0, NQ>([&](auto Cc) {
+    constexpr int c = decltype(Cc)::value;
+    static_for<0, NQ>([&](auto Rc) {
+      constexpr int r = decltype(Rc)::value;
+      out.minv(r, c, float(r <= c ? Mi[r][c] : Mi[c][r]));
+    });
+  });
+}
+
 // Full path for one knot in one lane.  P: arithmetic precision per phase.
 template <class P = PrecFP32, class In, class Out>
 RBD_HD RBD_INLINE void fdgrad_knot(const In& in, Out& out, const Options& opt) {
-  PhaseC<typename P::Col> PC;
-  typename P::Rnea qdd[NQ];
-  phase_a<P>(in, opt, PC, qdd);
+  using SM = typename P::Minv; using SR = typename P::Rnea; using SC = typename P::Col;
+  CS<KnotTrig<P>> tw[NQ];
+  knot_trig<P>(in, tw);
+  MassFactors<SM> f;
+  SR v[NQ][6], a[NQ][6], qdd[NQ];
+  knot_forward_dynamics<P>(in, opt, tw, f, v, a, qdd);
+  if constexpr (WantsMinv<Out>::value) {
+    store_minv(out, f);
+    if constexpr (StagesMinv<Out>::value) out.minv_done();
+  }
   for (int r = 0; r < NQ; ++r) out.qdd(r, float(qdd[r]));
-  if constexpr (WantsMinv<Out>::value)
-    for (int r = 0; r < NQ; ++r)
-      for (int c = 0; c < NQ; ++c) out.minv(r, c, float(r <= c ? PC.Mi[r][c] : PC.Mi[c][r]));
-  gradient_columns(PC, opt.damping, out);
+  CS<SR> tr[NQ];
+  cast_trig(tw, tr);
+  add_joint_accelerations(tr, qdd, a);
+  const TimesMassInverse<SM> times{f};
+  if constexpr (std::is_same<SR, SC>::value) {
+    gradient_columns(in, tr, v, a, opt.damping, times, out);
+  } else {
+    CS<SC> tc[NQ];
+    SC vc[NQ][6], ac[NQ][6];
+    cast_trig(tw, tc);
+    for (int k = 0; k < NQ; ++k)
+      for (int i = 0; i < 6; ++i) { vc[k][i] = SC(v[k][i]); ac[k][i] = SC(a[k][i]); }
+    gradient_columns(in, tc, vc, ac, opt.damping, times, out);
+  }
 }
 
 // Forward dynamics only: qdd = FD(q, qd, u) and the dense Minv, one lane per
@@ -945,30 +1395,14 @@ RBD_HD RBD_INLINE void fdgrad_knot(const In& in, Out& out, const Options& opt) {
 // with the bias RNEA at qdd = 0).
 template <class P = PrecFP32, class In, class Out>
 RBD_HD RBD_INLINE void fd_knot(const In& in, Out& out, const Options& opt) {
-  using SM = typename P::Minv; using SP = typename P::Pivot; using SR = typename P::Rnea;
-  using ST = Wider<SM, SR>;
-  CS<SM> tm[NQ]; CS<SR> tr[NQ];
-  SR qd[NQ], u[NQ];
-  for (int k = 0; k < NQ; ++k) {
-    ST s, c;
-    knot_sincos<P>(ST(in.q(k)), &s, &c);
-    tm[k] = CS<SM>{SM(c), SM(s)}; tr[k] = CS<SR>{SR(c), SR(s)};
-    qd[k] = SR(in.qd(k));
-    u[k] = SR(in.u(k));
-  }
-  SM Mi[NQ][NQ];
-  compute_minv<SM, SP>(tm, Mi);
-  SR v[NQ][6], a[NQ][6], f[NQ][6];
-  const SR zero[NQ] = {SR(0), SR(0), SR(0), SR(0), SR(0), SR(0), SR(0)};
-  rnea_fwd(tr, qd, zero, SR(opt.gravity), v, a, f);
-  subtract_fext(in, f);
-  rnea_bwd(tr, f);
-  SR bias[NQ], qdd[NQ];
-  for (int k = 0; k < NQ; ++k) bias[k] = u[k] - f[k][2] - SR(opt.damping) * qd[k];
-  minv_times<false>(Mi, bias, qdd);
+  using SM = typename P::Minv; using SR = typename P::Rnea;
+  CS<KnotTrig<P>> tw[NQ];
+  knot_trig<P>(in, tw);
+  MassFactors<SM> f;
+  SR v[NQ][6], a[NQ][6], qdd[NQ];
+  knot_forward_dynamics<P>(in, opt, tw, f, v, a, qdd);
   for (int r = 0; r < NQ; ++r) out.qdd(r, float(qdd[r]));
-  for (int r = 0; r < NQ; ++r)
-    for (int c = 0; c < NQ; ++c) out.minv(r, c, float(r <= c ? Mi[r][c] : Mi[c][r]));
+  store_minv(out, f);
 }
 
 // Minv of a knot shared by its lane group: the packed upper triangle
@@ -1159,7 +1593,7 @@ RBD_HD RBD_INLINE void two_wave_r1b(const Options& opt, int role, const TwoWaveR
   for (int r = 0; r < NQ; ++r)
     for (int c = 0; c < NQ; ++c) Mz[r][c] = SR(0);
   PhaseC<SC> PC;
-  make_phase_c(PC, st.tc, st.qd, st.v, st.a, st.f, Mz);
+  make_phase_c(PC, st.tc, st.v, st.a, st.f, Mz);
   const bool dq = role >= NQ;
   const int c = dq ? role - (NQ - 1) : role;
   dtau_column_uniform(PC, c, dq, tau_col);
@@ -1254,11 +1688,34 @@ RBD_HD RBD_INLINE void two_wave_r2(int role, const TwoWaveShared<P>& sh, typenam
 // qdd and a dense Minv are inputs; out is dqdd/dq, dqdd/dqd.  The upper triangle
 // of the given Minv is read (the same matrix for the symmetric Minv that
 // forwardDynamics produces).
+template <class P, class In, class Out, class Times>
+RBD_HD RBD_INLINE void gradient_given_qdd(const In& in, Out& out, const Options& opt, const Times& times) {
+  using SR = typename P::Rnea; using SC = typename P::Col;
+  CS<Wider<SR, SC>> tw[NQ];
+  knot_trig_in(P{}, in, tw);
+  CS<SR> tr[NQ];
+  cast_trig(tw, tr);
+  SR v[NQ][6], a[NQ][6], qd[NQ], qdd[NQ];
+  for (int k = 0; k < NQ; ++k) { qd[k] = SR(in.qd(k)); qdd[k] = SR(in.qdd(k)); }
+  link_motion(tr, qd, qdd, SR(opt.gravity), v, a);
+  if constexpr (std::is_same<SR, SC>::value) {
+    gradient_columns(in, tr, v, a, opt.damping, times, out);
+  } else {
+    CS<SC> tc[NQ];
+    SC vc[NQ][6], ac[NQ][6];
+    cast_trig(tw, tc);
+    for (int k = 0; k < NQ; ++k)
+      for (int i = 0; i < 6; ++i) { vc[k][i] = SC(v[k][i]); ac[k][i] = SC(a[k][i]); }
+    gradient_columns(in, tc, vc, ac, opt.damping, times, out);
+  }
+}
 template <class P = PrecFP32, class In, class Out>
 RBD_HD RBD_INLINE void fdgrad_knot_given_qdd_minv(const In& in, Out& out, const Options& opt) {
-  PhaseC<typename P::Col> PC;
-  phase_a_given_qdd_minv<P>(in, opt, PC);
-  gradient_columns(PC, opt.damping, out);
+  using SC = typename P::Col;
+  SC Mi[NQ][NQ];
+  for (int r = 0; r < NQ; ++r)
+    for (int c = r; c < NQ; ++c) Mi[r][c] = SC(in.minv(r, c));
+  gradient_given_qdd<P>(in, out, opt, TimesMinv<SC>{Mi});
 }
 
 // The same spread over a lane group.
@@ -1277,9 +1734,7 @@ RBD_HD RBD_INLINE void fdgrad_knot_given_qdd_minv_lanes(const In& in, Out& out, 
 // RNEA at qdd, then the derivative sweeps; no Minv.
 template <class P = PrecFP32, class In, class Out>
 RBD_HD RBD_INLINE void id_gradient_knot(const In& in, Out& out, const Options& opt) {
-  PhaseC<typename P::Col> PC;
-  phase_a_given_qdd_minv<P, false>(in, opt, PC);
-  gradient_columns<false>(PC, opt.damping, out);
+  gradient_given_qdd<P>(in, out, opt, TimesNothing{});
 }
 template <class P = PrecFP32, class In, class Out>
 RBD_HD RBD_INLINE void id_gradient_knot_lanes(const In& in, Out& out, const Options& opt, int role) {
@@ -1297,22 +1752,23 @@ template <class P, class In>
 RBD_HD RBD_INLINE void phase_split(const In& in, PhaseC<typename P::Col>& PC) {
   using SC = typename P::Col;
   CS<SC> tc[NQ];
-  SC qd[NQ], v[NQ][6], a[NQ][6], f[NQ][6], Mi[NQ][NQ];
+  SC v[NQ][6], a[NQ][6], f[NQ][6], Mi[NQ][NQ];
+  knot_trig_in(P{}, in, tc);
   for (int k = 0; k < NQ; ++k) {
-    SC s, c;
-    knot_sincos<P>(SC(in.q(k)), &s, &c);
-    tc[k] = CS<SC>{c, s};
-    qd[k] = SC(in.qd(k));
     for (int i = 0; i < 6; ++i) { v[k][i] = SC(in.v(k, i)); a[k][i] = SC(in.a(k, i)); f[k][i] = SC(in.f(k, i)); }
     for (int c2 = 0; c2 < NQ; ++c2) Mi[k][c2] = SC(0);
   }
-  make_phase_c(PC, tc, qd, v, a, f, Mi);
+  make_phase_c(PC, tc, v, a, f, Mi);
 }
 template <class P = PrecFP32, class In, class Out>
 RBD_HD RBD_INLINE void id_gradient_split_knot(const In& in, Out& out, const Options& opt) {
-  PhaseC<typename P::Col> PC;
-  phase_split<P>(in, PC);
-  gradient_columns<false>(PC, opt.damping, out);
+  using SC = typename P::Col;
+  CS<SC> tc[NQ];
+  knot_trig_in(P{}, in, tc);
+  SC v[NQ][6], a[NQ][6];
+  for (int k = 0; k < NQ; ++k)
+    for (int i = 0; i < 6; ++i) { v[k][i] = SC(in.v(k, i)); a[k][i] = SC(in.a(k, i)); }
+  gradient_columns<true>(in, tc, v, a, opt.damping, TimesNothing{}, out);
 }
 template <class P = PrecFP32, class In, class Out>
 RBD_HD RBD_INLINE void id_gradient_split_knot_lanes(const In& in, Out& out, const Options& opt, int role) {
@@ -1331,10 +1787,8 @@ RBD_HD RBD_INLINE void vaf_knot(const In& in, Out& out, const Options& opt) {
   using SR = typename P::Rnea;
   CS<SR> tr[NQ];
   SR qd[NQ], qdd[NQ];
+  knot_trig_in(P{}, in, tr);
   for (int k = 0; k < NQ; ++k) {
-    SR s, c;
-    knot_sincos<P>(SR(in.q(k)), &s, &c);
-    tr[k] = CS<SR>{c, s};
     qd[k] = SR(in.qd(k));
     qdd[k] = SR(in.qdd(k));
   }

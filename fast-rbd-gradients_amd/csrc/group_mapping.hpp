@@ -109,6 +109,7 @@ RBD_HD RBD_INLINE void group_stage2(const In& in, Out& out, const Options& opt, 
   phase_a_after_minv<P>(in, opt, tw, Mi, PC, qdd);
   static_for<0, Group<L>::kRounds>([&](auto Tc) {
     constexpr int t = decltype(Tc)::value;
+    if constexpr (t > 0) PC.link.forget();
     const int task = role + t * L;                 // 0..6 d/dqd c; 7..12 d/dq c - 6; 13 qdd; more: nothing
     if (task == kRoleQdd) {
       for (int r = 0; r < NQ; ++r) out.qdd(r, float(qdd[r]));

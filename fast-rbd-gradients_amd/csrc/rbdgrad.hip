@@ -102,9 +102,9 @@ __global__ __launch_bounds__(kBlock, kWavesPerSimd<P>) void fdgrad_aos_kernel(lo
 // (non-temporal) stores: each store writes one output row for the wave's 64
 // consecutive knots, 256 contiguous bytes, written once.  At 2^20 knots the
 // kernel measured 162 against 186 us with plain stores, whose write-allocated
-// lines kept the waves waiting.  The last column computed (d/dqd column 6,
-// the record's last 7 rows) is kept in `last` instead of stored: the kernel
-// stores it after the next knot's input loads have issued.
+// lines kept the waves waiting.  The last column computed (d/dqd column 0;
+// the columns come from the tip's to the base's) is kept in `last` instead of
+// stored: the kernel stores it after the next knot's input loads have issued.
 struct OutSoAStream {
   float* p; long ld;
   float* last;
@@ -112,7 +112,7 @@ struct OutSoAStream {
   __device__ void qdd(int i, float x) const { st(i, x); }
   __device__ void dq(int r, int c, float x) const { st(NQ + NQ * c + r, x); }
   __device__ void dqd(int r, int c, float x) const {
-    if (c == NQ - 1) last[r] = x;
+    if (c == 0) last[r] = x;
     else st(NQ + NQ * NQ + NQ * c + r, x);
   }
 };
@@ -126,7 +126,7 @@ struct OutSoAStream {
 template <class P>
 __global__ __launch_bounds__(kBlock, kWavesPerSimd<P>) void fdgrad_soa_kernel(long n, const float* __restrict__ in, long ld_in,
                                                             float* __restrict__ out, long ld_out, Options opt) {
-  constexpr int kLastRow = kOutPerKnot - NQ;
+  constexpr int kLastRow = NQ + NQ * NQ;     // d/dqd column 0
   const long stride = long(gridDim.x) * blockDim.x;
   float last[NQ];
   long prev = -1;
