@@ -302,6 +302,20 @@ __global__ __launch_bounds__(kMaxGroupWaves * kBlock, 1) void fdgrad_group_kerne
   }
 }
 
+// Output of a one-lane wave with Minv: Minv's 49 floats of each knot go into
+// the wave's record block and out to memory before the knot's record is
+// written there.
+struct OutAoSMinvStaged : OutAoS {
+  static constexpr bool kMinv = true;
+  float* block; float* minv_out; int words; int lane;
+  __device__ void minv(int r, int c, float x) const { block[NQ * NQ * lane + NQ * c + r] = x; }
+  __device__ void minv_done() const {
+    wave_lds_sync();
+    copy_record_block<true>(block, minv_out, words, lane);
+    wave_lds_sync();
+  }
+};
+
 // Full path plus dqdd/du = Minv (49 per knot, dense), both mappings.  WAFR:
 // out receives the WAFR baseline's 147-float layout (OutWafr) and minv is the
 // optional qdd buffer.
@@ -311,22 +325,26 @@ __global__ __launch_bounds__(kBlock, kWavesPerSimd<P>) void fdgrad_minv_kernel(l
                                                              Options opt) {
   using O = typename std::conditional<WAFR, OutWafr, OutAoSMinv>::type;
   if constexpr (LANES == 1) {
-    // the wave's 64 consecutive knots: both outputs staged in LDS, each copied
-    // out as one contiguous block (as fdgrad_aos_kernel does), by one round of
-    // resident waves: at 2^20 knots 252 against 385 us (+ Minv) and 252
-    // against 444 us (WAFR layout) with per-lane stores and a wave per block.
-    // The two blocks (39,424 bytes) leave a CU 4 waves.
+    // the wave's 64 consecutive knots: the outputs staged in LDS and copied out
+    // as contiguous blocks (as fdgrad_aos_kernel does), by one round of
+    // resident waves, each block's input loads issued before the previous
+    // block's copy.  + Minv: Minv goes through the record block first and is
+    // copied out before the gradient takes its place, so that the LDS holds
+    // one block of 26,880 bytes and a CU runs 6 waves (4 with a block of its
+    // own for Minv).  WAFR layout: Minv is part of the 147-float record (and
+    // qdd has a block of its own), which leaves a CU 4 waves.
     constexpr int kRec = WAFR ? kWafrPerKnot : kOutPerKnot;
-    constexpr int kAux = WAFR ? NQ : NQ * NQ;     // qdd (WAFR, optional) or Minv per knot
     __shared__ __align__(16) float rec[64 * kRec];
-    __shared__ __align__(16) float aux[64 * kAux];
-    // Each iteration issues its block's input loads before it copies out the
-    // previous block's records, as fdgrad_aos_kernel does: 236 against 252 us
-    // for either output, with bitwise the same results.
+    __shared__ __align__(16) float qrec[WAFR ? 64 * NQ : 1];
     const int lane = int(threadIdx.x);
     const long stride = long(gridDim.x) * kBlock;
-    long prev = 0;          // first knot of the block whose records rec, aux hold
+    long prev = 0;          // first knot of the block whose records rec, qrec hold
     int prev_nk = 0;        // and their knots (0: none yet)
+    auto copy_out = [&] {
+      copy_record_block<true>(rec, out + prev * kRec, prev_nk * kRec, lane);
+      if constexpr (WAFR)
+        if (minv) copy_record_block<true>(qrec, minv + prev * NQ, prev_nk * NQ, lane);
+    };
     for (long k0 = long(blockIdx.x) * kBlock; k0 < n; k0 += stride) {
       const int nk = int(n - k0 < kBlock ? n - k0 : kBlock);
       // lanes past the last knot compute a copy of it; only nk knots are written out
@@ -334,19 +352,20 @@ __global__ __launch_bounds__(kBlock, kWavesPerSimd<P>) void fdgrad_minv_kernel(l
       InRegs i;
       for (int j = 0; j < kInPerKnot; ++j) i.x[j] = src[j];
       __builtin_amdgcn_sched_barrier(0);
-      copy_record_block<true>(rec, out + prev * kRec, prev_nk * kRec, lane);
-      if (minv) copy_record_block<true>(aux, minv + prev * kAux, prev_nk * kAux, lane);
+      copy_out();
       __builtin_amdgcn_sched_barrier(0);
-      O o;
-      if constexpr (WAFR) o = OutWafr{minv ? aux + kAux * lane : nullptr, rec + kRec * lane};
-      else o = OutAoSMinv{rec + kRec * lane, aux + kAux * lane};
-      fdgrad_knot<P>(i, o, opt);
+      if constexpr (WAFR) {
+        OutWafr o{minv ? qrec + NQ * lane : nullptr, rec + kRec * lane};
+        fdgrad_knot<P>(i, o, opt);
+      } else {
+        OutAoSMinvStaged o{{rec + kRec * lane}, rec, minv + k0 * NQ * NQ, nk * NQ * NQ, lane};
+        fdgrad_knot<P>(i, o, opt);
+      }
       wave_lds_sync();
       prev = k0;
       prev_nk = nk;
     }
-    copy_record_block<true>(rec, out + prev * kRec, prev_nk * kRec, lane);
-    if (minv) copy_record_block<true>(aux, minv + prev * kAux, prev_nk * kAux, lane);
+    copy_out();
   } else {
     const int role = threadIdx.x % LANES;
     __shared__ typename P::Minv mi_sh[kBlock / kLanesPerKnotGroup][kMinvPacked];   // Minv per lane group
@@ -368,12 +387,13 @@ __global__ __launch_bounds__(kBlock, kWavesPerSimd<P>) void fdgrad_fext_kernel(l
                                                              const float* __restrict__ fext, long fext_stride,
                                                              float* __restrict__ out, Options opt) {
   if constexpr (LANES == 1) {
-    // records staged in LDS and copied out whole, as fdgrad_aos_kernel does
-    // by one round of resident waves (2^20 knots: 181 against 273 us with
-    // per-lane stores and a wave per block)
-    // (q, qd, u issued before the previous block's copy, as fdgrad_aos_kernel
-    // does; the forces are read where the RNEA needs them): 186 against 191 us
-    // with one set of forces per knot, bitwise the same results
+    // records staged in LDS and copied out whole, the inputs and forces issued
+    // before the previous block's copy, as fdgrad_aos_kernel does.  The bias
+    // pass and the derivative pass both need the 42 forces: they are kept in
+    // the knot's own record, floats 56..97, which the derivative pass writes
+    // column by column from the tip, each link's forces read before a column
+    // takes their place.
+    constexpr int kFextAt = NQ + NQ * NQ;                  // d/dqd column 0
     __shared__ __align__(16) float rec[kRecordBlockFloats];
     const int lane = int(threadIdx.x);
     const long stride = long(gridDim.x) * kBlock;
@@ -383,12 +403,17 @@ __global__ __launch_bounds__(kBlock, kWavesPerSimd<P>) void fdgrad_fext_kernel(l
       const int nk = int(n - k0 < kBlock ? n - k0 : kBlock);
       const long k = k0 + (lane < nk ? lane : nk - 1);
       const float* src = in + kInPerKnot * k;
+      const float* fsrc = fext + fext_stride * k;
       InRegs i;
+      float fx[kFextPerSet];
       for (int j = 0; j < kInPerKnot; ++j) i.x[j] = src[j];
-      i.fx = fext + fext_stride * k;
+      for (int j = 0; j < kFextPerSet; ++j) fx[j] = fsrc[j];
       __builtin_amdgcn_sched_barrier(0);
       copy_record_block<true>(rec, out + prev * kOutPerKnot, prev_words, lane);
       __builtin_amdgcn_sched_barrier(0);
+      wave_lds_sync();
+      for (int j = 0; j < kFextPerSet; ++j) rec[kOutPerKnot * lane + kFextAt + j] = fx[j];
+      i.fx = rec + kOutPerKnot * lane + kFextAt;
       OutAoS o{rec + kOutPerKnot * lane};
       fdgrad_knot<P>(i, o, opt);
       wave_lds_sync();
@@ -435,40 +460,139 @@ __global__ __launch_bounds__(kBlock, kWavesPerSimd<P>) void fd_kernel(long n, co
   }
 }
 
+// 16-byte pieces of a wave's block of 64 records of F floats, piece 64 j + lane
+// in x[j]; the block must be whole and 16-byte aligned.
+typedef float v4f __attribute__((ext_vector_type(4)));
+template <int F> constexpr int kBlockPieces = 64 * F / 4;
+template <int F> constexpr int kLanePieces = (kBlockPieces<F> + 63) / 64;
+template <int F>
+__device__ RBD_INLINE void load_block(const float* src, int lane, v4f x[kLanePieces<F>]) {
+  static_for<0, kLanePieces<F>>([&](auto Jc) {
+    constexpr int j = decltype(Jc)::value;
+    if (64 * j + 63 < kBlockPieces<F> || lane < kBlockPieces<F> - 64 * j)
+      x[j] = reinterpret_cast<const v4f*>(src)[64 * j + lane];
+  });
+}
+template <int F>
+__device__ RBD_INLINE void put_block(const v4f x[kLanePieces<F>], int lane, float* rec) {
+  static_for<0, kLanePieces<F>>([&](auto Jc) {
+    constexpr int j = decltype(Jc)::value;
+    if (64 * j + 63 < kBlockPieces<F> || lane < kBlockPieces<F> - 64 * j)
+      reinterpret_cast<v4f*>(rec)[64 * j + lane] = x[j];
+  });
+}
+
+// q, qd, qdd of a 28-float record, in registers
+struct InFusedRegs {
+  float x[3 * NQ];
+  const float* fx = nullptr;
+  __device__ void load(const float* p) {
+#pragma unroll
+    for (int k = 0; k < NQ; ++k) {
+      x[k] = p[k];
+      x[NQ + k] = p[NQ + k];
+      x[2 * NQ + k] = p[3 * NQ + k];
+    }
+  }
+  __device__ float q(int i) const { return x[i]; }
+  __device__ float qd(int i) const { return x[NQ + i]; }
+  __device__ float qdd(int i) const { return x[2 * NQ + i]; }
+};
+
+// The precisions whose one-lane inverse-dynamics gradient stages its records
+// in LDS: FP32 columns (with FP64 columns the lanes read and write their own).
+template <class P> constexpr bool kStagedIdGradient = sizeof(typename P::Col) == 4 && sizeof(typename P::Rnea) == 4;
+
 // Inverse-dynamics gradient (cdu, 98 per knot) from q, qd, qdd (SPLIT = false:
 // 28 per knot, the fused layout) or from q, qd and precomputed v, a, f
 // (SPLIT = true: 154 per knot, the split layout).  Both mappings.
 template <class P, int LANES, bool SPLIT>
 __global__ __launch_bounds__(kBlock, kWavesPerSimd<P>) void id_gradient_kernel(long n, const float* __restrict__ vol,
                                                              float* __restrict__ cdu, Options opt) {
-  if constexpr (LANES == 1 && SPLIT && std::is_same<P, PrecFP32>::value) {
+  if constexpr (LANES == 1 && SPLIT && kStagedIdGradient<P>) {
     // FP32, split layout: the wave's 64 consecutive input records (154 floats
     // each, one contiguous block) are read into LDS as whole lines, 16 bytes
     // per lane, and each lane then reads its record from there.  Read by each
-    // lane at the 616-byte record stride, they were fetched 5x over.
-    typedef float v4f __attribute__((ext_vector_type(4)));
-    __shared__ __align__(16) float inrec[64 * kSplitPerKnot];
+    // lane at the 616-byte record stride, they were fetched 5x over.  The
+    // lane's 98 outputs go over the first 98 floats of its own record (q, qd,
+    // u, qdd, v and part of a, which the lane has read by then; f lies above
+    // them), and the wave copies them out in whole lines: stored by each lane
+    // from its registers they wrote 1.9x their bytes.  LDS holds one block, so
+    // a CU runs 4 waves.  The next block's loads are issued before the copy.
+    typedef float v2f __attribute__((ext_vector_type(2)));
+    __shared__ __align__(16) float rec[64 * kSplitPerKnot];
     const int lane = int(threadIdx.x);
     const long stride = long(gridDim.x) * kBlock;
+    long prev = 0;          // first knot of the block whose outputs rec holds
+    int prev_nk = 0;        // and their knots (0: none yet)
+    auto copy_out = [&] {
+      float* dst = cdu + prev * kDqddPerKnot;
+      if ((reinterpret_cast<uintptr_t>(dst) & 7u) == 0) {
+        constexpr int kPairs = kDqddPerKnot / 2;                       // 49 pairs per record
+        int r = lane / kPairs, c = lane % kPairs;
+        for (int e = lane; e < prev_nk * kPairs; e += 64) {
+          put<true>(reinterpret_cast<v2f*>(dst) + e, *reinterpret_cast<const v2f*>(rec + kSplitPerKnot * r + 2 * c));
+          r += 1;                                                      // 64 = 49 + 15
+          c += 64 - kPairs;
+          if (c >= kPairs) { c -= kPairs; r += 1; }
+        }
+      } else {
+        for (int e = lane; e < prev_nk * kDqddPerKnot; e += 64)
+          put<true>(dst + e, rec[kSplitPerKnot * (e / kDqddPerKnot) + e % kDqddPerKnot]);
+      }
+    };
     for (long k0 = long(blockIdx.x) * kBlock; k0 < n; k0 += stride) {
       const int nk = int(n - k0 < kBlock ? n - k0 : kBlock);
       const float* src = vol + k0 * kSplitPerKnot;
-      const int words = nk * kSplitPerKnot;
-      if ((reinterpret_cast<uintptr_t>(src) & 15u) == 0) {
-        for (int e = lane; e < words / 4; e += 64)
-          reinterpret_cast<v4f*>(inrec)[e] = reinterpret_cast<const v4f*>(src)[e];
-        for (int e = (words / 4) * 4 + lane; e < words; e += 64) inrec[e] = src[e];
+      if (nk == kBlock && (reinterpret_cast<uintptr_t>(src) & 15u) == 0) {
+        v4f x[kLanePieces<kSplitPerKnot>];
+        load_block<kSplitPerKnot>(src, lane, x);
+        __builtin_amdgcn_sched_barrier(0);
+        copy_out();
+        wave_lds_sync();
+        put_block<kSplitPerKnot>(x, lane, rec);
       } else {
-        for (int e = lane; e < words; e += 64) inrec[e] = src[e];
+        copy_out();
+        wave_lds_sync();
+        for (int e = lane; e < nk * kSplitPerKnot; e += 64) rec[e] = src[e];
       }
       wave_lds_sync();
       if (lane < nk) {
-        InSplit i{inrec + kSplitPerKnot * lane};
-        OutDqddAoS o{cdu + kDqddPerKnot * (k0 + lane)};
+        InSplit i{rec + kSplitPerKnot * lane};
+        OutDqddAoS o{rec + kSplitPerKnot * lane};
         id_gradient_split_knot<P>(i, o, opt);
       }
-      wave_lds_sync();                      // every lane has read its record before the next block overwrites inrec
+      wave_lds_sync();
+      prev = k0;
+      prev_nk = nk;
     }
+    copy_out();
+    return;
+  }
+  if constexpr (LANES == 1 && !SPLIT && kStagedIdGradient<P>) {
+    // FP32, fused layout: outputs staged in LDS and copied out whole, each
+    // block's inputs loaded before the previous block's copy, as in
+    // fdgrad_refmode_kernel
+    __shared__ __align__(16) float rec[kDqddBlockFloats];
+    const int lane = int(threadIdx.x);
+    const long stride = long(gridDim.x) * kBlock;
+    long prev = 0;          // first knot of the block whose records rec holds
+    int prev_words = 0;     // and their words (0: none yet)
+    for (long k0 = long(blockIdx.x) * kBlock; k0 < n; k0 += stride) {
+      const int nk = int(n - k0 < kBlock ? n - k0 : kBlock);
+      // lanes past the last knot compute a copy of it; only nk records are written out
+      InFusedRegs i;
+      i.load(vol + kFusedPerKnot * (k0 + (lane < nk ? lane : nk - 1)));
+      __builtin_amdgcn_sched_barrier(0);
+      copy_record_block<true>(rec, cdu + prev * kDqddPerKnot, prev_words, lane);
+      __builtin_amdgcn_sched_barrier(0);
+      OutDqddAoS o{rec + kDqddPerKnot * lane};
+      id_gradient_knot<P>(i, o, opt);
+      wave_lds_sync();
+      prev = k0;
+      prev_words = nk * kDqddPerKnot;
+    }
+    copy_record_block<true>(rec, cdu + prev * kDqddPerKnot, prev_words, lane);
     return;
   }
   const int role = threadIdx.x % LANES;
@@ -523,25 +647,66 @@ __global__ __launch_bounds__(kBlock, kWavesPerSimd<P>) void vaf_kernel(long n, f
   }
 }
 
-// dqdd = -Minv cdu per knot.  One lane per knot; the wave's 64 consecutive
-// knots' results are staged in LDS and copied out as one contiguous block of
-// 64 x 98 floats, as fdgrad_refmode_kernel does.
-__global__ __launch_bounds__(kBlock) void finish_kernel(long n, const float* __restrict__ minv,
-                                                        const float* __restrict__ cdu, float* __restrict__ dqdd) {
+// Minv in registers (its upper triangle) and a cdu record
+struct InFinishRegs {
+  const float (*m)[NQ]; const float* c;
+  __device__ float minv(int r, int col) const { return m[r][col]; }
+  __device__ float cdu(int r, int col) const { return c[r + NQ * col]; }
+};
+
+// dqdd = -Minv cdu per knot, one lane per knot.  Bound by memory (980 bytes per
+// knot in and out): the wave's blocks of 64 Minv (49 floats) and 64 cdu (98)
+// are read as whole lines into registers, all loads in flight at once, and
+// handed to the lanes through one LDS block in turn, Minv first; each lane's
+// results take the place of its cdu and leave as whole lines.  Read by each
+// lane at the record strides, every line was fetched about four times from the
+// L2.  A block that is short or not 16-byte aligned goes through LDS float by
+// float.
+__global__ __launch_bounds__(kBlock, 2) void finish_kernel(long n, const float* __restrict__ minv,
+                                                           const float* __restrict__ cdu, float* __restrict__ dqdd) {
   __shared__ __align__(16) float rec[kDqddBlockFloats];
   const int lane = int(threadIdx.x);
   const long stride = long(gridDim.x) * kBlock;
+  long prev = 0;          // first knot of the block whose results rec holds
+  int prev_words = 0;     // and their words (0: none yet)
   for (long k0 = long(blockIdx.x) * kBlock; k0 < n; k0 += stride) {
     const int nk = int(n - k0 < kBlock ? n - k0 : kBlock);
-    // lanes past the last knot compute a copy of it; only nk records are written out
-    const long k = k0 + (lane < nk ? lane : nk - 1);
-    InFinish i{minv + NQ * NQ * k, cdu + kDqddPerKnot * k};
+    const float* msrc = minv + NQ * NQ * k0;
+    const float* csrc = cdu + kDqddPerKnot * k0;
+    const bool whole = nk == kBlock && ((reinterpret_cast<uintptr_t>(msrc) | reinterpret_cast<uintptr_t>(csrc)) & 15u) == 0;
+    v4f m4[kLanePieces<NQ * NQ>], c4[kLanePieces<kDqddPerKnot>];
+    if (whole) {
+      load_block<NQ * NQ>(msrc, lane, m4);
+      load_block<kDqddPerKnot>(csrc, lane, c4);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    copy_record_block<true>(rec, dqdd + prev * kDqddPerKnot, prev_words, lane);
+    __builtin_amdgcn_sched_barrier(0);
+    wave_lds_sync();
+    if (whole) put_block<NQ * NQ>(m4, lane, rec);
+    else for (int e = lane; e < nk * NQ * NQ; e += 64) rec[e] = msrc[e];
+    wave_lds_sync();
+    // lanes past the last knot read what the block holds and store nothing that is copied out
+    float Mi[NQ][NQ];
+    static_for<0, NQ>([&](auto Rc) {
+      constexpr int r = decltype(Rc)::value;
+      static_for<r, NQ>([&](auto Cc) {
+        constexpr int c = decltype(Cc)::value;
+        Mi[r][c] = rec[NQ * NQ * lane + r + NQ * c];
+      });
+    });
+    wave_lds_sync();
+    if (whole) put_block<kDqddPerKnot>(c4, lane, rec);
+    else for (int e = lane; e < nk * kDqddPerKnot; e += 64) rec[e] = csrc[e];
+    wave_lds_sync();
+    InFinishRegs i{Mi, rec + kDqddPerKnot * lane};
     OutFinish o{rec + kDqddPerKnot * lane};
     finish_knot(i, o);
     wave_lds_sync();
-    copy_record_block<true>(rec, dqdd + k0 * kDqddPerKnot, nk * kDqddPerKnot, lane);
-    wave_lds_sync();                        // read out before the next knots overwrite rec
+    prev = k0;
+    prev_words = nk * kDqddPerKnot;
   }
+  copy_record_block<true>(rec, dqdd + prev * kDqddPerKnot, prev_words, lane);
 }
 
 }  // namespace rbd
@@ -1096,11 +1261,16 @@ rbd_status id_gradient(rbd_context* ctx, int64_t n, float* d_cdu, const float* d
   const int lanes = lanes_for(ctx, n);
   const dim3 grid(grid_for(n, lanes)), block(kBlock);
   const hipStream_t st = (hipStream_t)stream;
+  hipError_t ge = hipSuccess;
   auto go = [&](auto prec_tag) {
     using P = decltype(prec_tag);
-    if (lanes == 1)
-      hipLaunchKernelGGL((rbd::id_gradient_kernel<P, 1, SPLIT>), grid, block, 0, st, long(n), d_vol, d_cdu, ctx->opt);
-    else
+    if (lanes == 1) {
+      dim3 g = grid;
+      if constexpr (rbd::kStagedIdGradient<P>)
+        ge = one_lane_grid<rbd::id_gradient_kernel<P, 1, SPLIT>>(ctx->compute_units, &g);
+      if (ge == hipSuccess)
+        hipLaunchKernelGGL((rbd::id_gradient_kernel<P, 1, SPLIT>), g, block, 0, st, long(n), d_vol, d_cdu, ctx->opt);
+    } else
       hipLaunchKernelGGL((rbd::id_gradient_kernel<P, rbd::kLanesPerKnotGroup, SPLIT>), grid, block, 0, st, long(n),
                          d_vol, d_cdu, ctx->opt);
   };
@@ -1111,6 +1281,7 @@ rbd_status id_gradient(rbd_context* ctx, int64_t n, float* d_cdu, const float* d
     case RBD_PREC_FP64_COLUMNS: go(rbd::PrecFP64Col{}); break;
     default: go(rbd::PrecFP64{}); break;
   }
+  if (ge != hipSuccess) return hip_fail(ge, "occupancy query");
   hipError_t e = hipGetLastError();
   return e == hipSuccess ? RBD_OK : hip_fail(e, "id_gradient_kernel launch");
 }
@@ -1155,7 +1326,8 @@ rbd_status rbd_gradient_finish_f32(rbd_context* ctx, int64_t n, float* d_dqdd, c
   if (n == 0) return RBD_OK;
   if (!d_dqdd || !d_cdu || !d_minv) return fail(RBD_ERR_INVALID_ARGUMENT, "null buffer");
   if (rbd_status s = ready_to_launch(ctx)) return s;
-  const dim3 grid(grid_for(n, 1)), block(kBlock);
+  dim3 grid(grid_for(n, 1)), block(kBlock);
+  if (hipError_t ge = one_lane_grid<rbd::finish_kernel>(ctx->compute_units, &grid)) return hip_fail(ge, "occupancy query");
   hipLaunchKernelGGL(rbd::finish_kernel, grid, block, 0, (hipStream_t)stream, long(n), d_minv, d_cdu, d_dqdd);
   hipError_t e = hipGetLastError();
   return e == hipSuccess ? RBD_OK : hip_fail(e, "finish_kernel launch");
