@@ -61,16 +61,120 @@ template <typename S> struct CS { S c, s; };
 RBD_HD RBD_INLINE float fma_s(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 RBD_HD RBD_INLINE double fma_s(double a, double b, double c) { return __builtin_fma(a, b, c); }
 
-RBD_HD RBD_INLINE void sincos_s(float x, float* s, float* c) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  ::sincosf(x, s, c);
-#else
-  *s = std::sin(x); *c = std::cos(x);
-#endif
+// sin and cos without divergent branches.  The math library's take one path
+// for ordinary arguments and another for huge ones, an if/else that lanes may
+// split over; in kernels short of registers the compiler moved values that
+// live across it into accumulation registers or scratch at the start of the
+// block where the two paths meet, ahead of the instruction that turns the
+// other lanes back on, so that with no lane on the rare path nothing was saved
+// and garbage came back (in FP64-column kernels: wrong gradients in groups of
+// 8 lanes, stores to garbage addresses).  Below, every lane takes one straight
+// path, and a second one only if some lane of the wave is out of its range.
+//
+// r = x - k pi/2 in [-pi/4, pi/4], sin and cos of r by minimax polynomials in
+// r^2 fitted for that range, quadrant k mod 4.
+//
+// FP32, |x| <= 512: pi/2 in three parts.  The first difference is exact; the
+// second part has 15 bits, so that its product with k (9 bits) is exact too
+// and what rounding r loses can be formed, and goes into the results with the
+// third part as the low word lo.  Polynomial errors 3.6e-9 and 1e-10; the
+// results are within 0.92 units in the last place.
+template <typename S> constexpr S kSincosMax = sizeof(S) == 4 ? S(512) : S(65536);
+RBD_HD RBD_INLINE void sincos_reduced(float x, float* s, float* c) {
+  const float k = __builtin_rintf(x * 0.63661977236758134f);
+  const float r1 = __builtin_fmaf(-k, 0x1.921fb6p+0f, x);
+  const float r = __builtin_fmaf(-k, -0x1.777cp-25f, r1);
+  // what rounding r lost, and the third part
+  const float lo = __builtin_fmaf(-k, 0x1.a308d4p-41f, __builtin_fmaf(-k, -0x1.777cp-25f, r1 - r));
+  const float z = r * r;
+  float ps = __builtin_fmaf(z, -0x1.994b4p-13f, 0x1.110756p-7f);
+  ps = __builtin_fmaf(z, ps, -0x1.555546p-3f);
+  const float sr = r + __builtin_fmaf(r * z, ps, lo);
+  float pc = __builtin_fmaf(z, 0x1.99ff42p-16f, -0x1.6c0c82p-10f);
+  pc = __builtin_fmaf(z, pc, 0x1.55554ap-5f);
+  const float hz = 0.5f * z, ca = 1.0f - hz;
+  const float cr = ca + __builtin_fmaf(z * z, pc, __builtin_fmaf(-lo, r, (1.0f - ca) - hz));
+  const unsigned q = unsigned(int(k));
+  const bool swap = (q & 1u) != 0u;
+  const float ss = swap ? cr : sr, cc = swap ? sr : cr;
+  *s = (q & 2u) ? -ss : ss;
+  *c = ((q + 1u) & 2u) ? -cc : cc;
 }
-RBD_HD RBD_INLINE void sincos_s(double x, double* s, double* c) {
+// sin and cos of q pi/2 + r in FP64 (polynomial errors 3.5e-18 and 4.7e-20)
+RBD_HD RBD_INLINE void sincos_quadrant(unsigned q, double r, double* s, double* c) {
+  const double z = r * r;
+  double ps = __builtin_fma(z, 0x1.5d92451b64143p-33, -0x1.ae5e63c6fd08dp-26);
+  ps = __builtin_fma(z, ps, 0x1.71de3574b0c8ap-19);
+  ps = __builtin_fma(z, ps, -0x1.a01a019c0e3efp-13);
+  ps = __builtin_fma(z, ps, 0x1.111111110f861p-7);
+  ps = __builtin_fma(z, ps, -0x1.5555555555549p-3);
+  const double sr = __builtin_fma(r * z, ps, r);
+  double pc = __builtin_fma(z, -0x1.8fadd03da3e34p-37, 0x1.1ee9ea6c52bd8p-29);
+  pc = __builtin_fma(z, pc, -0x1.27e4f807d5628p-22);
+  pc = __builtin_fma(z, pc, 0x1.a01a019caef23p-16);
+  pc = __builtin_fma(z, pc, -0x1.6c16c16c15162p-10);
+  pc = __builtin_fma(z, pc, 0x1.555555555554cp-5);
+  const double cr = __builtin_fma(z, __builtin_fma(z, pc, -0.5), 1.0);
+  const bool swap = (q & 1u) != 0u;
+  const double ss = swap ? cr : sr, cc = swap ? sr : cr;
+  *s = (q & 2u) ? -ss : ss;
+  *c = ((q + 1u) & 2u) ? -cc : cc;
+}
+// FP64, |x| <= 65536: pi/2 in two parts (results within 2 units in the last
+// place; every output is FP32)
+RBD_HD RBD_INLINE void sincos_reduced(double x, double* s, double* c) {
+  const double k = __builtin_rint(x * 0x1.45f306dc9c883p-1);
+  const double r = __builtin_fma(-k, 0x1.1a62633145c07p-54, __builtin_fma(-k, 0x1.921fb54442d18p+0, x));
+  sincos_quadrant(unsigned(int(k)), r, s, c);
+}
+// sin and cos of an FP32 angle of any size from 2^-7 up, by integer arithmetic
+// (Payne and Hanek's reduction): with x = m 2^E, the bits of 2/pi from weight
+// 2^(1 - E) on, as a 128-bit number W, give x 2/pi mod 4 = (m W mod 2^128)
+// 2^-126: two bits of quadrant and 126 of fraction, of which an FP32 x cancels
+// at most about 30.
+RBD_HD RBD_INLINE void sincos_far(float x, double* s, double* c) {
+  constexpr unsigned kTwoOverPi[9] = {0u, 0xa2f9836eu, 0x4e441529u, 0xfc2757d1u, 0xf534ddc0u, 0xdb629599u, 0x3c439041u, 0xfe5163abu, 0xdebbc561u};
+  const unsigned bits = __builtin_bit_cast(unsigned, x);
+  const unsigned m = (bits & 0x7fffffu) | 0x800000u;
+  const int e = int((bits >> 23) & 255u) - 120;      // first bit of W, after 32 zero bits
+  const unsigned p = unsigned(e < 0 ? 0 : e), word = p >> 5, shift = p & 31u;
+  unsigned w[5];                                     // the five words that W lies in
+  static_for<0, 5>([&](auto Jc) {
+    constexpr int j = decltype(Jc)::value;
+    w[j] = kTwoOverPi[j];
+    static_for<1, 5>([&](auto Kc) {
+      constexpr int k = decltype(Kc)::value;
+      w[j] = word == unsigned(k) ? kTwoOverPi[j + k] : w[j];
+    });
+  });
+  unsigned long long t = 0;
+  unsigned limb[4];
+  static_for_down<4, 0>([&](auto Jc) {
+    constexpr int j = decltype(Jc)::value;
+    const unsigned long long two = (static_cast<unsigned long long>(w[j]) << 32) | w[j + 1];
+    t = static_cast<unsigned long long>(m) * unsigned(two >> (32u - shift)) + (t >> 32);
+    limb[j] = unsigned(t);
+  });
+  const unsigned long long hi = (static_cast<unsigned long long>(limb[0]) << 32) | limb[1];
+  const unsigned long long lo = (static_cast<unsigned long long>(limb[2]) << 32) | limb[3];
+  const unsigned q = unsigned((hi + (1ull << 61)) >> 62);           // nearest quarter turn
+  const double f = double(static_cast<long long>(hi - (static_cast<unsigned long long>(q) << 62))) + double(lo) * 0x1p-64;
+  const double r = f * (0x1p-62 * 0x1.921fb54442d18p+0);
+  const bool neg = (bits >> 31) != 0u;
+  sincos_quadrant(neg ? 0u - q : q, neg ? -r : r, s, c);
+}
+// sin and cos of a joint angle x (an FP32 value in either type)
+template <typename S>
+RBD_HD RBD_INLINE void sincos_s(S x, S* s, S* c) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  ::sincos(x, s, c);
+  sincos_reduced(x, s, c);
+  const bool far = !(__builtin_fabs(x) <= kSincosMax<S>);
+  if (__ballot(far) != 0) {              // the same in every lane
+    double sf, cf;
+    sincos_far(float(x), &sf, &cf);
+    *s = far ? S(sf) : *s;
+    *c = far ? S(cf) : *c;
+  }
 #else
   *s = std::sin(x); *c = std::cos(x);
 #endif
