@@ -52,50 +52,47 @@ using rbdi::kBlock;
 // ---------------------------------------------------------------------------
 namespace rbd {
 
-// One lane per knot, array-of-structures, records staged in LDS.  A wave takes
-// 64 consecutive knots, whose 105-float records are one contiguous block of
-// 26,880 bytes: each lane writes its record into LDS at the record's own
-// stride (105 floats, odd: no bank conflicts), and the wave copies the block
-// out with consecutive lanes on consecutive 16-byte pieces, so each store
-// covers 1 KB of contiguous output (8 cache lines) instead of 64 records'
-// lines.  Per-lane record stores had the cache and address units stalling the
-// waves (at 2^20 knots: 5.2x the L1 accesses and 4.9x the L2 write requests
-// of the structure-of-arrays layout).  The block limits a CU to 6 waves.  The
-// copy uses streaming (non-temporal) stores.
-//
-// A wave's vector-memory counter retires loads and stores in the order they
-// were issued, so waiting for a block's input loads also waits for every store
-// issued before them.  Each loop iteration therefore issues its block's loads
-// first and only then copies out the previous block's records (2^20 knots:
-// 179.5-181.4 against 183.3-184.9 us).  The copy's LDS reads precede the next
-// records' LDS writes in program order, on the same array, and a wave's LDS
-// operations execute in order, so no fence separates them; a fence there
-// changed how the compiler contracted the knot's products into FMAs, and with
-// it the results' last bits.
+// F contiguous floats in 16-byte pieces over the wave, piece 64 j + lane in
+// x[j]; 16-byte aligned.
+typedef float v4f __attribute__((ext_vector_type(4)));
+template <int F> constexpr int kBlockPieces = F / 4;
+template <int F> constexpr int kLanePieces = (kBlockPieces<F> + 63) / 64;
+template <int F>
+__device__ RBD_INLINE void load_block(const float* src, int lane, v4f x[kLanePieces<F>]) {
+  static_for<0, kLanePieces<F>>([&](auto Jc) {
+    constexpr int j = decltype(Jc)::value;
+    if (64 * j + 63 < kBlockPieces<F> || lane < kBlockPieces<F> - 64 * j)
+      x[j] = reinterpret_cast<const v4f*>(src)[64 * j + lane];
+  });
+}
+template <int F>
+__device__ RBD_INLINE void put_block(const v4f x[kLanePieces<F>], int lane, float* rec) {
+  static_for<0, kLanePieces<F>>([&](auto Jc) {
+    constexpr int j = decltype(Jc)::value;
+    if (64 * j + 63 < kBlockPieces<F> || lane < kBlockPieces<F> - 64 * j)
+      reinterpret_cast<v4f*>(rec)[64 * j + lane] = x[j];
+  });
+}
+
+// A knot's 21 inputs from its record
+__device__ RBD_INLINE void load_inputs(const float* src, InRegs& i) {
+  for (int j = 0; j < kInPerKnot; ++j) i.x[j] = src[j];
+}
+
+// One lane per knot, array-of-structures, records through LDS (records.hpp).
+// Per-lane record stores had the cache and address units stalling the waves
+// (at 2^20 knots: 5.2x the L1 accesses and 4.9x the L2 write requests of the
+// structure-of-arrays layout).
 template <class P>
 __global__ __launch_bounds__(kBlock, kWavesPerSimd<P>) void fdgrad_aos_kernel(long n, const float* __restrict__ in,
                                                             float* __restrict__ out, Options opt) {
-  __shared__ __align__(16) float rec[kRecordBlockFloats];
-  const int lane = int(threadIdx.x);
-  const long stride = long(gridDim.x) * kBlock;
-  long prev = 0;          // first knot of the block whose records rec holds
-  int prev_words = 0;     // and their words (0: none yet)
-  for (long k0 = long(blockIdx.x) * kBlock; k0 < n; k0 += stride) {
-    const int nk = int(n - k0 < kBlock ? n - k0 : kBlock);
-    // lanes past the last knot compute a copy of it; only nk records are written out
-    const float* src = in + kInPerKnot * (k0 + (lane < nk ? lane : nk - 1));
-    InRegs i;
-    for (int j = 0; j < kInPerKnot; ++j) i.x[j] = src[j];
-    __builtin_amdgcn_sched_barrier(0);
-    copy_record_block<true>(rec, out + prev * kOutPerKnot, prev_words, lane);
-    __builtin_amdgcn_sched_barrier(0);
-    OutAoS o{rec + kOutPerKnot * lane};
-    fdgrad_knot<P>(i, o, opt);
-    wave_lds_sync();
-    prev = k0;
-    prev_words = nk * kOutPerKnot;
-  }
-  copy_record_block<true>(rec, out + prev * kOutPerKnot, prev_words, lane);
+  __shared__ __align__(16) float rec[kRecordLds<P, kOutPerKnot>];
+  one_lane_records<P, kOutPerKnot, InRegs>(
+      n, out, rec, [&](long k, InRegs& i) { load_inputs(in + kInPerKnot * k, i); },
+      [&](const InRegs& i, float* p, long, int) {
+        OutAoS o{p};
+        fdgrad_knot<P>(i, o, opt);
+      });
 }
 
 // Structure-of-arrays output of the one-lane kernel with streaming
@@ -145,21 +142,14 @@ __global__ __launch_bounds__(kBlock, kWavesPerSimd<P>) void fdgrad_soa_kernel(lo
     for (int r = 0; r < NQ; ++r) put<true>(out + (kLastRow + r) * ld_out + prev, last[r]);
 }
 
-// Reference-compatible mode (qdd and Minv given), one lane per knot: a wave's
-// 64 consecutive knots write one contiguous block of 64 x 98 floats, staged in
-// LDS and copied out whole as in the AoS kernel above: 215.6 us at 2^20
-// knots, against 381 us with per-lane stores of the 98-float records.  As
-// there, each iteration issues its block's input loads (the 49 of a record's
-// 77 floats the gradient reads: q, qd, qdd and Minv's upper triangle) before
-// it copies out the previous block's records: 200 against 216-218 us, with
-// the same FP instruction mix and bitwise the same results.
+// Reference-compatible mode (qdd and Minv given), one lane per knot, records
+// through LDS.  The gradient reads 49 of a record's 77 floats: q, qd, qdd and
+// Minv's upper triangle.
 constexpr int kDqddBlockFloats = 64 * kDqddPerKnot;
 struct InVolRegs {
-  static constexpr int kUpper = NQ * (NQ + 1) / 2;
-  float x[3 * NQ + kUpper];
+  float x[3 * NQ];
+  float m[NQ][NQ];
   const float* fx = nullptr;
-  // row r of the upper triangle starts at r * NQ - r * (r - 1) / 2
-  static constexpr int upper(int r, int c) { return 3 * NQ + r * NQ - r * (r - 1) / 2 + (c - r); }
   __device__ void load(const float* p) {
 #pragma unroll
     for (int k = 0; k < NQ; ++k) {
@@ -167,40 +157,33 @@ struct InVolRegs {
       x[NQ + k] = p[NQ + k];
       x[2 * NQ + k] = p[3 * NQ + k];
     }
+  }
+  __device__ void load_minv(const float* p) {
 #pragma unroll
     for (int r = 0; r < NQ; ++r)
 #pragma unroll
-      for (int c = r; c < NQ; ++c) x[upper(r, c)] = p[4 * NQ + r + NQ * c];
+      for (int c = r; c < NQ; ++c) m[r][c] = p[4 * NQ + r + NQ * c];
   }
   __device__ float q(int i) const { return x[i]; }
   __device__ float qd(int i) const { return x[NQ + i]; }
   __device__ float qdd(int i) const { return x[2 * NQ + i]; }
-  __device__ float minv(int r, int c) const { return x[upper(r, c)]; }   // r <= c: only the upper triangle is read
+  __device__ float minv(int r, int c) const { return m[r][c]; }   // r <= c: only the upper triangle is read
 };
 
 template <class P>
 __global__ __launch_bounds__(kBlock, kWavesPerSimd<P>) void fdgrad_refmode_kernel(long n, const float* __restrict__ vol,
                                                                 float* __restrict__ dqdd, Options opt) {
-  __shared__ __align__(16) float rec[kDqddBlockFloats];
-  const int lane = int(threadIdx.x);
-  const long stride = long(gridDim.x) * kBlock;
-  long prev = 0;          // first knot of the block whose records rec holds
-  int prev_words = 0;     // and their words (0: none yet)
-  for (long k0 = long(blockIdx.x) * kBlock; k0 < n; k0 += stride) {
-    const int nk = int(n - k0 < kBlock ? n - k0 : kBlock);
-    // lanes past the last knot compute a copy of it; only nk records are written out
-    InVolRegs i;
-    i.load(vol + kVolPerKnot * (k0 + (lane < nk ? lane : nk - 1)));
-    __builtin_amdgcn_sched_barrier(0);
-    copy_record_block<true>(rec, dqdd + prev * kDqddPerKnot, prev_words, lane);
-    __builtin_amdgcn_sched_barrier(0);
-    OutDqddAoS o{rec + kDqddPerKnot * lane};
-    fdgrad_knot_given_qdd_minv<P>(i, o, opt);
-    wave_lds_sync();
-    prev = k0;
-    prev_words = nk * kDqddPerKnot;
-  }
-  copy_record_block<true>(rec, dqdd + prev * kDqddPerKnot, prev_words, lane);
+  __shared__ __align__(16) float rec[kRecordLds<P, kDqddPerKnot>];
+  one_lane_records<P, kDqddPerKnot, InVolRegs>(
+      n, dqdd, rec, [&](long k, InVolRegs& i) { i.load(vol + kVolPerKnot * k); },
+      [&](InVolRegs& i, float* p, long k0, int nk) {
+        // Minv is first needed by the last product of the tip's column, long
+        // after it has arrived; loaded with the rest, it would have to share
+        // the registers with the previous block's outputs
+        i.load_minv(vol + kVolPerKnot * (k0 + min(int(threadIdx.x), nk - 1)));
+        OutDqddAoS o{p};
+        fdgrad_knot_given_qdd_minv<P>(i, o, opt);
+      });
 }
 
 // One knot per group of kLanesPerKnotGroup lanes (4 knots per wave): the
@@ -325,47 +308,31 @@ __global__ __launch_bounds__(kBlock, kWavesPerSimd<P>) void fdgrad_minv_kernel(l
                                                              Options opt) {
   using O = typename std::conditional<WAFR, OutWafr, OutAoSMinv>::type;
   if constexpr (LANES == 1) {
-    // the wave's 64 consecutive knots: the outputs staged in LDS and copied out
-    // as contiguous blocks (as fdgrad_aos_kernel does), by one round of
-    // resident waves, each block's input loads issued before the previous
-    // block's copy.  + Minv: Minv goes through the record block first and is
-    // copied out before the gradient takes its place, so that the LDS holds
-    // one block of 26,880 bytes and a CU runs 6 waves (4 with a block of its
-    // own for Minv).  WAFR layout: Minv is part of the 147-float record (and
-    // qdd has a block of its own), which leaves a CU 4 waves.
+    // + Minv: Minv goes through the record LDS first and is copied out before
+    // the gradient takes its place, so that it takes no LDS of its own.  WAFR
+    // layout: Minv is part of the 147-float record, and qdd has a block of its
+    // own.
     constexpr int kRec = WAFR ? kWafrPerKnot : kOutPerKnot;
-    __shared__ __align__(16) float rec[64 * kRec];
+    __shared__ __align__(16) float rec[kRecordLds<P, kRec>];
     __shared__ __align__(16) float qrec[WAFR ? 64 * NQ : 1];
+    static_assert(kRecordLds<P, kOutPerKnot> >= 64 * NQ * NQ, "Minv of 64 knots");
     const int lane = int(threadIdx.x);
-    const long stride = long(gridDim.x) * kBlock;
-    long prev = 0;          // first knot of the block whose records rec, qrec hold
-    int prev_nk = 0;        // and their knots (0: none yet)
-    auto copy_out = [&] {
-      copy_record_block<true>(rec, out + prev * kRec, prev_nk * kRec, lane);
-      if constexpr (WAFR)
-        if (minv) copy_record_block<true>(qrec, minv + prev * NQ, prev_nk * NQ, lane);
-    };
-    for (long k0 = long(blockIdx.x) * kBlock; k0 < n; k0 += stride) {
-      const int nk = int(n - k0 < kBlock ? n - k0 : kBlock);
-      // lanes past the last knot compute a copy of it; only nk knots are written out
-      const float* src = in + kInPerKnot * (k0 + (lane < nk ? lane : nk - 1));
-      InRegs i;
-      for (int j = 0; j < kInPerKnot; ++j) i.x[j] = src[j];
-      __builtin_amdgcn_sched_barrier(0);
-      copy_out();
-      __builtin_amdgcn_sched_barrier(0);
-      if constexpr (WAFR) {
-        OutWafr o{minv ? qrec + NQ * lane : nullptr, rec + kRec * lane};
-        fdgrad_knot<P>(i, o, opt);
-      } else {
-        OutAoSMinvStaged o{{rec + kRec * lane}, rec, minv + k0 * NQ * NQ, nk * NQ * NQ, lane};
-        fdgrad_knot<P>(i, o, opt);
-      }
-      wave_lds_sync();
-      prev = k0;
-      prev_nk = nk;
-    }
-    copy_out();
+    one_lane_records<P, kRec, InRegs>(
+        n, out, rec, [&](long k, InRegs& i) { load_inputs(in + kInPerKnot * k, i); },
+        [&](const InRegs& i, float* p, long k0, int nk) {
+          if constexpr (WAFR) {
+            OutWafr o{minv ? qrec + NQ * lane : nullptr, p};
+            fdgrad_knot<P>(i, o, opt);
+            if (minv) {
+              wave_lds_sync();
+              copy_record_block<true>(qrec, minv + k0 * NQ, nk * NQ, lane);
+              wave_lds_sync();
+            }
+          } else {
+            OutAoSMinvStaged o{{p}, rec, minv + k0 * NQ * NQ, nk * NQ * NQ, lane};
+            fdgrad_knot<P>(i, o, opt);
+          }
+        });
   } else {
     const int role = threadIdx.x % LANES;
     __shared__ typename P::Minv mi_sh[kBlock / kLanesPerKnotGroup][kMinvPacked];   // Minv per lane group
@@ -387,40 +354,28 @@ __global__ __launch_bounds__(kBlock, kWavesPerSimd<P>) void fdgrad_fext_kernel(l
                                                              const float* __restrict__ fext, long fext_stride,
                                                              float* __restrict__ out, Options opt) {
   if constexpr (LANES == 1) {
-    // records staged in LDS and copied out whole, the inputs and forces issued
-    // before the previous block's copy, as fdgrad_aos_kernel does.  The bias
-    // pass and the derivative pass both need the 42 forces: they are kept in
-    // the knot's own record, floats 56..97, which the derivative pass writes
-    // column by column from the tip, each link's forces read before a column
-    // takes their place.
-    constexpr int kFextAt = NQ + NQ * NQ;                  // d/dqd column 0
-    __shared__ __align__(16) float rec[kRecordBlockFloats];
-    const int lane = int(threadIdx.x);
-    const long stride = long(gridDim.x) * kBlock;
-    long prev = 0;          // first knot of the block whose records rec holds
-    int prev_words = 0;     // and their words (0: none yet)
-    for (long k0 = long(blockIdx.x) * kBlock; k0 < n; k0 += stride) {
-      const int nk = int(n - k0 < kBlock ? n - k0 : kBlock);
-      const long k = k0 + (lane < nk ? lane : nk - 1);
-      const float* src = in + kInPerKnot * k;
-      const float* fsrc = fext + fext_stride * k;
-      InRegs i;
-      float fx[kFextPerSet];
-      for (int j = 0; j < kInPerKnot; ++j) i.x[j] = src[j];
-      for (int j = 0; j < kFextPerSet; ++j) fx[j] = fsrc[j];
-      __builtin_amdgcn_sched_barrier(0);
-      copy_record_block<true>(rec, out + prev * kOutPerKnot, prev_words, lane);
-      __builtin_amdgcn_sched_barrier(0);
-      wave_lds_sync();
-      for (int j = 0; j < kFextPerSet; ++j) rec[kOutPerKnot * lane + kFextAt + j] = fx[j];
-      i.fx = rec + kOutPerKnot * lane + kFextAt;
-      OutAoS o{rec + kOutPerKnot * lane};
-      fdgrad_knot<P>(i, o, opt);
-      wave_lds_sync();
-      prev = k0;
-      prev_words = nk * kOutPerKnot;
-    }
-    copy_record_block<true>(rec, out + prev * kOutPerKnot, prev_words, lane);
+    // The bias pass and the derivative pass both need the 42 forces: they are
+    // kept in the record LDS between the two.  With outputs in registers that
+    // LDS is free until they are complete (stride 43 floats: odd); else they
+    // lie in the knot's own record, floats 56..97, which the derivative pass
+    // writes column by column from the tip, each link's forces read before a
+    // column takes their place.
+    constexpr int kFextAt = kHoldOutputs<P> ? 0 : NQ + NQ * NQ;      // d/dqd column 0
+    constexpr int kFextStride = kHoldOutputs<P> ? kFextPerSet + 1 : kOutPerKnot;
+    __shared__ __align__(16) float rec[kRecordLds<P, kOutPerKnot>];
+    static_assert(kRecordLds<P, kOutPerKnot> >= 64 * (kFextPerSet + 1), "forces of 64 knots");
+    float* mine = rec + kFextStride * int(threadIdx.x) + kFextAt;
+    one_lane_records<P, kOutPerKnot, InRegs>(
+        n, out, rec, [&](long k, InRegs& i) { load_inputs(in + kInPerKnot * k, i); },
+        [&](InRegs& i, float* p, long k0, int nk) {
+          const float* f = fext + fext_stride * (k0 + min(int(threadIdx.x), nk - 1));
+          float fx[kFextPerSet];
+          for (int j = 0; j < kFextPerSet; ++j) fx[j] = f[j];
+          for (int j = 0; j < kFextPerSet; ++j) mine[j] = fx[j];
+          i.fx = mine;
+          OutAoS o{p};
+          fdgrad_knot<P>(i, o, opt);
+        });
   } else {
     const int role = threadIdx.x % LANES;
     __shared__ typename P::Minv mi_sh[kBlock / kLanesPerKnotGroup][kMinvPacked];   // Minv per lane group
@@ -460,28 +415,6 @@ __global__ __launch_bounds__(kBlock, kWavesPerSimd<P>) void fd_kernel(long n, co
   }
 }
 
-// 16-byte pieces of a wave's block of 64 records of F floats, piece 64 j + lane
-// in x[j]; the block must be whole and 16-byte aligned.
-typedef float v4f __attribute__((ext_vector_type(4)));
-template <int F> constexpr int kBlockPieces = 64 * F / 4;
-template <int F> constexpr int kLanePieces = (kBlockPieces<F> + 63) / 64;
-template <int F>
-__device__ RBD_INLINE void load_block(const float* src, int lane, v4f x[kLanePieces<F>]) {
-  static_for<0, kLanePieces<F>>([&](auto Jc) {
-    constexpr int j = decltype(Jc)::value;
-    if (64 * j + 63 < kBlockPieces<F> || lane < kBlockPieces<F> - 64 * j)
-      x[j] = reinterpret_cast<const v4f*>(src)[64 * j + lane];
-  });
-}
-template <int F>
-__device__ RBD_INLINE void put_block(const v4f x[kLanePieces<F>], int lane, float* rec) {
-  static_for<0, kLanePieces<F>>([&](auto Jc) {
-    constexpr int j = decltype(Jc)::value;
-    if (64 * j + 63 < kBlockPieces<F> || lane < kBlockPieces<F> - 64 * j)
-      reinterpret_cast<v4f*>(rec)[64 * j + lane] = x[j];
-  });
-}
-
 // q, qd, qdd of a 28-float record, in registers
 struct InFusedRegs {
   float x[3 * NQ];
@@ -499,9 +432,27 @@ struct InFusedRegs {
   __device__ float qdd(int i) const { return x[2 * NQ + i]; }
 };
 
+struct InNothing {};
+
+// q, v, a, f of a 154-float record, in registers
+struct InSplitRegs {
+  float x[NQ + 18 * NQ];
+  const float* fx = nullptr;
+  __device__ void load(const float* p) {
+#pragma unroll
+    for (int k = 0; k < NQ; ++k) x[k] = p[k];
+#pragma unroll
+    for (int k = 0; k < 18 * NQ; ++k) x[NQ + k] = p[4 * NQ + k];
+  }
+  __device__ float q(int i) const { return x[i]; }
+  __device__ float v(int k, int i) const { return x[NQ + 6 * k + i]; }
+  __device__ float a(int k, int i) const { return x[7 * NQ + 6 * k + i]; }
+  __device__ float f(int k, int i) const { return x[13 * NQ + 6 * k + i]; }
+};
+
 // The precisions whose one-lane inverse-dynamics gradient stages its records
 // in LDS: FP32 columns (with FP64 columns the lanes read and write their own).
-template <class P> constexpr bool kStagedIdGradient = sizeof(typename P::Col) == 4 && sizeof(typename P::Rnea) == 4;
+template <class P> constexpr bool kStagedIdGradient = kHoldOutputs<P>;
 
 // Inverse-dynamics gradient (cdu, 98 per knot) from q, qd, qdd (SPLIT = false:
 // 28 per knot, the fused layout) or from q, qd and precomputed v, a, f
@@ -510,89 +461,48 @@ template <class P, int LANES, bool SPLIT>
 __global__ __launch_bounds__(kBlock, kWavesPerSimd<P>) void id_gradient_kernel(long n, const float* __restrict__ vol,
                                                              float* __restrict__ cdu, Options opt) {
   if constexpr (LANES == 1 && SPLIT && kStagedIdGradient<P>) {
-    // FP32, split layout: the wave's 64 consecutive input records (154 floats
-    // each, one contiguous block) are read into LDS as whole lines, 16 bytes
-    // per lane, and each lane then reads its record from there.  Read by each
-    // lane at the 616-byte record stride, they were fetched 5x over.  The
-    // lane's 98 outputs go over the first 98 floats of its own record (q, qd,
-    // u, qdd, v and part of a, which the lane has read by then; f lies above
-    // them), and the wave copies them out in whole lines: stored by each lane
-    // from its registers they wrote 1.9x their bytes.  LDS holds one block, so
-    // a CU runs 4 waves.  The next block's loads are issued before the copy.
-    typedef float v2f __attribute__((ext_vector_type(2)));
-    __shared__ __align__(16) float rec[64 * kSplitPerKnot];
+    // FP32 columns, split layout: the wave's 64 consecutive input records (154
+    // floats each) are read as whole lines, 32 at a time through LDS, from
+    // where each lane takes the 126 floats it needs into registers; the
+    // outputs leave through the same LDS (records.hpp).  Read by each lane at
+    // the 616-byte record stride, the inputs were fetched 5x over, and outputs
+    // stored by each lane wrote 1.9x their bytes.
+    __shared__ __align__(16) float rec[32 * kSplitPerKnot];
     const int lane = int(threadIdx.x);
-    const long stride = long(gridDim.x) * kBlock;
-    long prev = 0;          // first knot of the block whose outputs rec holds
-    int prev_nk = 0;        // and their knots (0: none yet)
-    auto copy_out = [&] {
-      float* dst = cdu + prev * kDqddPerKnot;
-      if ((reinterpret_cast<uintptr_t>(dst) & 7u) == 0) {
-        constexpr int kPairs = kDqddPerKnot / 2;                       // 49 pairs per record
-        int r = lane / kPairs, c = lane % kPairs;
-        for (int e = lane; e < prev_nk * kPairs; e += 64) {
-          put<true>(reinterpret_cast<v2f*>(dst) + e, *reinterpret_cast<const v2f*>(rec + kSplitPerKnot * r + 2 * c));
-          r += 1;                                                      // 64 = 49 + 15
-          c += 64 - kPairs;
-          if (c >= kPairs) { c -= kPairs; r += 1; }
-        }
-      } else {
-        for (int e = lane; e < prev_nk * kDqddPerKnot; e += 64)
-          put<true>(dst + e, rec[kSplitPerKnot * (e / kDqddPerKnot) + e % kDqddPerKnot]);
-      }
-    };
-    for (long k0 = long(blockIdx.x) * kBlock; k0 < n; k0 += stride) {
-      const int nk = int(n - k0 < kBlock ? n - k0 : kBlock);
-      const float* src = vol + k0 * kSplitPerKnot;
-      if (nk == kBlock && (reinterpret_cast<uintptr_t>(src) & 15u) == 0) {
-        v4f x[kLanePieces<kSplitPerKnot>];
-        load_block<kSplitPerKnot>(src, lane, x);
-        __builtin_amdgcn_sched_barrier(0);
-        copy_out();
-        wave_lds_sync();
-        put_block<kSplitPerKnot>(x, lane, rec);
-      } else {
-        copy_out();
-        wave_lds_sync();
-        for (int e = lane; e < nk * kSplitPerKnot; e += 64) rec[e] = src[e];
-      }
-      wave_lds_sync();
-      if (lane < nk) {
-        InSplit i{rec + kSplitPerKnot * lane};
-        OutDqddAoS o{rec + kSplitPerKnot * lane};
-        id_gradient_split_knot<P>(i, o, opt);
-      }
-      wave_lds_sync();
-      prev = k0;
-      prev_nk = nk;
-    }
-    copy_out();
+    one_lane_records<P, kDqddPerKnot, InNothing>(
+        n, cdu, rec, [](long, InNothing&) {},
+        [&](const InNothing&, float* p, long k0, int nk) {
+          InSplitRegs i;
+          static_for<0, 2>([&](auto Hc) {
+            constexpr int h = decltype(Hc)::value;
+            const int left = nk - 32 * h;
+            const int words = (left < 0 ? 0 : left < 32 ? left : 32) * kSplitPerKnot;
+            const float* src = vol + (k0 + 32 * h) * kSplitPerKnot;
+            if (words == 32 * kSplitPerKnot && (reinterpret_cast<uintptr_t>(src) & 15u) == 0) {
+              v4f x[kLanePieces<32 * kSplitPerKnot>];
+              load_block<32 * kSplitPerKnot>(src, lane, x);
+              put_block<32 * kSplitPerKnot>(x, lane, rec);
+            } else {
+              for (int e = lane; e < words; e += 64) rec[e] = src[e];
+            }
+            wave_lds_sync();
+            // lanes past the last knot take what the LDS holds; nothing of theirs is written out
+            if ((lane >> 5) == h) i.load(rec + kSplitPerKnot * (lane & 31));
+            wave_lds_sync();
+          });
+          OutDqddAoS o{p};
+          id_gradient_split_knot<P>(i, o, opt);
+        });
     return;
   }
   if constexpr (LANES == 1 && !SPLIT && kStagedIdGradient<P>) {
-    // FP32, fused layout: outputs staged in LDS and copied out whole, each
-    // block's inputs loaded before the previous block's copy, as in
-    // fdgrad_refmode_kernel
-    __shared__ __align__(16) float rec[kDqddBlockFloats];
-    const int lane = int(threadIdx.x);
-    const long stride = long(gridDim.x) * kBlock;
-    long prev = 0;          // first knot of the block whose records rec holds
-    int prev_words = 0;     // and their words (0: none yet)
-    for (long k0 = long(blockIdx.x) * kBlock; k0 < n; k0 += stride) {
-      const int nk = int(n - k0 < kBlock ? n - k0 : kBlock);
-      // lanes past the last knot compute a copy of it; only nk records are written out
-      InFusedRegs i;
-      i.load(vol + kFusedPerKnot * (k0 + (lane < nk ? lane : nk - 1)));
-      __builtin_amdgcn_sched_barrier(0);
-      copy_record_block<true>(rec, cdu + prev * kDqddPerKnot, prev_words, lane);
-      __builtin_amdgcn_sched_barrier(0);
-      OutDqddAoS o{rec + kDqddPerKnot * lane};
-      id_gradient_knot<P>(i, o, opt);
-      wave_lds_sync();
-      prev = k0;
-      prev_words = nk * kDqddPerKnot;
-    }
-    copy_record_block<true>(rec, cdu + prev * kDqddPerKnot, prev_words, lane);
+    __shared__ __align__(16) float rec[kRecordLds<P, kDqddPerKnot>];
+    one_lane_records<P, kDqddPerKnot, InFusedRegs>(
+        n, cdu, rec, [&](long k, InFusedRegs& i) { i.load(vol + kFusedPerKnot * k); },
+        [&](const InFusedRegs& i, float* p, long, int) {
+          OutDqddAoS o{p};
+          id_gradient_knot<P>(i, o, opt);
+        });
     return;
   }
   const int role = threadIdx.x % LANES;
@@ -674,16 +584,16 @@ __global__ __launch_bounds__(kBlock, 2) void finish_kernel(long n, const float* 
     const float* msrc = minv + NQ * NQ * k0;
     const float* csrc = cdu + kDqddPerKnot * k0;
     const bool whole = nk == kBlock && ((reinterpret_cast<uintptr_t>(msrc) | reinterpret_cast<uintptr_t>(csrc)) & 15u) == 0;
-    v4f m4[kLanePieces<NQ * NQ>], c4[kLanePieces<kDqddPerKnot>];
+    v4f m4[kLanePieces<64 * NQ * NQ>], c4[kLanePieces<64 * kDqddPerKnot>];
     if (whole) {
-      load_block<NQ * NQ>(msrc, lane, m4);
-      load_block<kDqddPerKnot>(csrc, lane, c4);
+      load_block<64 * NQ * NQ>(msrc, lane, m4);
+      load_block<64 * kDqddPerKnot>(csrc, lane, c4);
     }
     __builtin_amdgcn_sched_barrier(0);
     copy_record_block<true>(rec, dqdd + prev * kDqddPerKnot, prev_words, lane);
     __builtin_amdgcn_sched_barrier(0);
     wave_lds_sync();
-    if (whole) put_block<NQ * NQ>(m4, lane, rec);
+    if (whole) put_block<64 * NQ * NQ>(m4, lane, rec);
     else for (int e = lane; e < nk * NQ * NQ; e += 64) rec[e] = msrc[e];
     wave_lds_sync();
     // lanes past the last knot read what the block holds and store nothing that is copied out
@@ -696,7 +606,7 @@ __global__ __launch_bounds__(kBlock, 2) void finish_kernel(long n, const float* 
       });
     });
     wave_lds_sync();
-    if (whole) put_block<kDqddPerKnot>(c4, lane, rec);
+    if (whole) put_block<64 * kDqddPerKnot>(c4, lane, rec);
     else for (int e = lane; e < nk * kDqddPerKnot; e += 64) rec[e] = csrc[e];
     wave_lds_sync();
     InFinishRegs i{Mi, rec + kDqddPerKnot * lane};

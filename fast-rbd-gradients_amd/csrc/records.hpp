@@ -1,10 +1,10 @@
 // Whole-record output through LDS for the one-lane-per-knot kernels (device
 // code).  A wave's 64 consecutive knots have one contiguous block of records
-// (64 x 105 floats = 26,880 bytes).  Each lane writes its record into an LDS
-// copy of that block (at the record stride of 105 floats, which is odd, so the
-// lanes' writes fall in different banks), and the wave then copies the block
-// out with consecutive lanes on consecutive 16-byte pieces: every store covers
-// 1 KB of contiguous output instead of 64 records' cache lines.
+// (64 x 105 floats = 26,880 bytes); the lanes hand their records over in LDS
+// (at the record stride, 105 floats: odd, so their writes fall in different
+// banks), and the wave copies them out with consecutive lanes on consecutive
+// 16-byte pieces: every store covers 1 KB of contiguous output instead of 64
+// records' cache lines.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -40,6 +40,62 @@ __device__ inline void copy_record_block(const float* rec, float* dst, int words
     for (int e = (words / 4) * 4 + lane; e < words; e += 64) put<NT>(dst + e, rec[e]);
   } else {
     for (int e = lane; e < words; e += 64) put<NT>(dst + e, rec[e]);
+  }
+}
+
+// Whether a one-lane kernel of precision P keeps a knot's outputs in registers
+// until they are complete: with FP32 columns they fit (255 registers, no
+// spills, two waves per SIMD: what the derivative pass no longer needs makes
+// room for them); with FP64 columns they go into LDS as they come.
+template <class P> constexpr bool kHoldOutputs = kWavesPerSimd<P> == 2;
+// Floats of LDS for records of REC floats
+template <class P, int REC> constexpr int kRecordLds = (kHoldOutputs<P> ? 32 : 64) * REC;
+
+// A one-lane kernel's loop over the wave's blocks of 64 knots with records of
+// REC floats: load(k, in) reads knot k's inputs into registers, compute(in, p,
+// k0, nk) computes the knot and stores its record at p, and the wave writes
+// the nk records of knots k0.. to out.
+//
+// With the outputs in registers, 32 records go through LDS at a time, so a
+// wave needs 13,440 bytes and a CU runs 8 waves; with the whole block in LDS
+// it ran 6 (2^20 knots: HOLD_NOTE).  The next block's loads are issued before
+// the copies: a wave's vector-memory counter retires loads and stores in the
+// order they were issued, so waiting for loads also waits for every store
+// issued before them.  Lanes past the last knot compute a copy of it; only nk
+// records are written out.  rec: kRecordLds<P, REC> floats or more, which
+// compute may use too until it returns.
+template <class P, int REC, class In, class Load, class Compute>
+__device__ RBD_INLINE void one_lane_records(long n, float* out, float* rec, Load&& load, Compute&& compute) {
+  const int lane = int(threadIdx.x);
+  const long stride = long(gridDim.x) * 64;
+  long k0 = long(blockIdx.x) * 64;
+  if (k0 >= n) return;
+  In in;
+  load(k0 + lane < n ? k0 + lane : n - 1, in);
+  for (; k0 < n; k0 += stride) {
+    const int nk = int(n - k0 < 64 ? n - k0 : 64);
+    float r[kHoldOutputs<P> ? REC : 1];
+    compute(in, kHoldOutputs<P> ? r : rec + REC * lane, k0, nk);
+    const long k1 = k0 + stride + lane;
+    if (k0 + stride < n) load(k1 < n ? k1 : n - 1, in);
+    __builtin_amdgcn_sched_barrier(0);
+    wave_lds_sync();
+    if constexpr (kHoldOutputs<P>) {
+      static_for<0, 2>([&](auto Hc) {
+        constexpr int h = decltype(Hc)::value;
+        if ((lane >> 5) == h) {
+          float* d = rec + REC * (lane & 31);
+          static_for<0, REC>([&](auto Jc) { d[decltype(Jc)::value] = r[decltype(Jc)::value]; });
+        }
+        wave_lds_sync();
+        const int left = nk - 32 * h;
+        copy_record_block<true>(rec, out + (k0 + 32 * h) * REC, (left < 0 ? 0 : left < 32 ? left : 32) * REC, lane);
+        wave_lds_sync();                    // read out before the next records overwrite it
+      });
+    } else {
+      copy_record_block<true>(rec, out + k0 * REC, nk * REC, lane);
+      wave_lds_sync();
+    }
   }
 }
 
