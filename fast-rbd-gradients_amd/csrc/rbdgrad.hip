@@ -52,28 +52,6 @@ using rbdi::kBlock;
 // ---------------------------------------------------------------------------
 namespace rbd {
 
-// F contiguous floats in 16-byte pieces over the wave, piece 64 j + lane in
-// x[j]; 16-byte aligned.
-typedef float v4f __attribute__((ext_vector_type(4)));
-template <int F> constexpr int kBlockPieces = F / 4;
-template <int F> constexpr int kLanePieces = (kBlockPieces<F> + 63) / 64;
-template <int F>
-__device__ RBD_INLINE void load_block(const float* src, int lane, v4f x[kLanePieces<F>]) {
-  static_for<0, kLanePieces<F>>([&](auto Jc) {
-    constexpr int j = decltype(Jc)::value;
-    if (64 * j + 63 < kBlockPieces<F> || lane < kBlockPieces<F> - 64 * j)
-      x[j] = reinterpret_cast<const v4f*>(src)[64 * j + lane];
-  });
-}
-template <int F>
-__device__ RBD_INLINE void put_block(const v4f x[kLanePieces<F>], int lane, float* rec) {
-  static_for<0, kLanePieces<F>>([&](auto Jc) {
-    constexpr int j = decltype(Jc)::value;
-    if (64 * j + 63 < kBlockPieces<F> || lane < kBlockPieces<F> - 64 * j)
-      reinterpret_cast<v4f*>(rec)[64 * j + lane] = x[j];
-  });
-}
-
 // A knot's 21 inputs from its record
 __device__ RBD_INLINE void load_inputs(const float* src, InRegs& i) {
   for (int j = 0; j < kInPerKnot; ++j) i.x[j] = src[j];
@@ -294,7 +272,7 @@ struct OutAoSMinvStaged : OutAoS {
   __device__ void minv(int r, int c, float x) const { block[NQ * NQ * lane + NQ * c + r] = x; }
   __device__ void minv_done() const {
     wave_lds_sync();
-    copy_record_block<true>(block, minv_out, words, lane);
+    copy_record_block<true, 64 * NQ * NQ>(block, minv_out, words, lane);
     wave_lds_sync();
   }
 };
@@ -310,11 +288,14 @@ __global__ __launch_bounds__(kBlock, kWavesPerSimd<P>) void fdgrad_minv_kernel(l
   if constexpr (LANES == 1) {
     // + Minv: Minv goes through the record LDS first and is copied out before
     // the gradient takes its place, so that it takes no LDS of its own.  WAFR
-    // layout: Minv is part of the 147-float record, and qdd has a block of its
-    // own.
+    // layout: Minv is part of the 147-float record, and qdd takes Minv's way (a
+    // block of its own beside the record's 18,816 bytes would leave room for 7
+    // waves per CU instead of 8: 131,000 knots 30.3 us against 25.0), with FP64
+    // columns a block of its own.
     constexpr int kRec = WAFR ? kWafrPerKnot : kOutPerKnot;
     __shared__ __align__(16) float rec[kRecordLds<P, kRec>];
-    __shared__ __align__(16) float qrec[WAFR ? 64 * NQ : 1];
+    __shared__ __align__(16) float qown[WAFR && !kHoldOutputs<P> ? 64 * NQ : 1];
+    float* qrec = kHoldOutputs<P> ? rec : qown;
     static_assert(kRecordLds<P, kOutPerKnot> >= 64 * NQ * NQ, "Minv of 64 knots");
     const int lane = int(threadIdx.x);
     one_lane_records<P, kRec, InRegs>(
@@ -325,7 +306,7 @@ __global__ __launch_bounds__(kBlock, kWavesPerSimd<P>) void fdgrad_minv_kernel(l
             fdgrad_knot<P>(i, o, opt);
             if (minv) {
               wave_lds_sync();
-              copy_record_block<true>(qrec, minv + k0 * NQ, nk * NQ, lane);
+              copy_record_block<true, 64 * NQ>(qrec, minv + k0 * NQ, nk * NQ, lane);
               wave_lds_sync();
             }
           } else {
@@ -409,8 +390,8 @@ __global__ __launch_bounds__(kBlock, kWavesPerSimd<P>) void fd_kernel(long n, co
     OutFD o{qrec + NQ * lane, mrec + NQ * NQ * lane};
     fd_knot<P>(i, o, opt);
     wave_lds_sync();
-    copy_record_block<true>(qrec, qdd + NQ * k0, nk * NQ, lane);
-    copy_record_block<true>(mrec, minv + NQ * NQ * k0, nk * NQ * NQ, lane);
+    copy_record_block<true, 64 * NQ>(qrec, qdd + NQ * k0, nk * NQ, lane);
+    copy_record_block<true, 64 * NQ * NQ>(mrec, minv + NQ * NQ * k0, nk * NQ * NQ, lane);
     wave_lds_sync();                        // read out before the next knots overwrite them
   }
 }
@@ -478,12 +459,10 @@ __global__ __launch_bounds__(kBlock, kWavesPerSimd<P>) void id_gradient_kernel(l
             const int left = nk - 32 * h;
             const int words = (left < 0 ? 0 : left < 32 ? left : 32) * kSplitPerKnot;
             const float* src = vol + (k0 + 32 * h) * kSplitPerKnot;
-            if (words == 32 * kSplitPerKnot && (reinterpret_cast<uintptr_t>(src) & 15u) == 0) {
-              v4f x[kLanePieces<32 * kSplitPerKnot>];
-              load_block<32 * kSplitPerKnot>(src, lane, x);
-              put_block<32 * kSplitPerKnot>(x, lane, rec);
-            } else {
-              for (int e = lane; e < words; e += 64) rec[e] = src[e];
+            if (words > 0) {
+              BlockPieces<32 * kSplitPerKnot> x;
+              load_block<32 * kSplitPerKnot>(src, words, lane, x);
+              put_block<32 * kSplitPerKnot>(x, words, lane, rec);
             }
             wave_lds_sync();
             // lanes past the last knot take what the LDS holds; nothing of theirs is written out
@@ -544,7 +523,7 @@ __global__ __launch_bounds__(kBlock, kWavesPerSimd<P>) void vaf_kernel(long n, f
       OutVaf o{r};
       vaf_knot<P>(i, o, opt);
       wave_lds_sync();
-      copy_record_block<true>(rec, vol + k0 * kSplitPerKnot, nk * kSplitPerKnot, lane);
+      copy_record_block<true, 64 * kSplitPerKnot>(rec, vol + k0 * kSplitPerKnot, nk * kSplitPerKnot, lane);
       wave_lds_sync();                      // read out before the next knots overwrite rec
     }
   } else {
@@ -570,8 +549,7 @@ struct InFinishRegs {
 // handed to the lanes through one LDS block in turn, Minv first; each lane's
 // results take the place of its cdu and leave as whole lines.  Read by each
 // lane at the record strides, every line was fetched about four times from the
-// L2.  A block that is short or not 16-byte aligned goes through LDS float by
-// float.
+// L2.
 __global__ __launch_bounds__(kBlock, 2) void finish_kernel(long n, const float* __restrict__ minv,
                                                            const float* __restrict__ cdu, float* __restrict__ dqdd) {
   __shared__ __align__(16) float rec[kDqddBlockFloats];
@@ -583,18 +561,15 @@ __global__ __launch_bounds__(kBlock, 2) void finish_kernel(long n, const float* 
     const int nk = int(n - k0 < kBlock ? n - k0 : kBlock);
     const float* msrc = minv + NQ * NQ * k0;
     const float* csrc = cdu + kDqddPerKnot * k0;
-    const bool whole = nk == kBlock && ((reinterpret_cast<uintptr_t>(msrc) | reinterpret_cast<uintptr_t>(csrc)) & 15u) == 0;
-    v4f m4[kLanePieces<64 * NQ * NQ>], c4[kLanePieces<64 * kDqddPerKnot>];
-    if (whole) {
-      load_block<64 * NQ * NQ>(msrc, lane, m4);
-      load_block<64 * kDqddPerKnot>(csrc, lane, c4);
-    }
+    BlockPieces<64 * NQ * NQ> m4;
+    BlockPieces<64 * kDqddPerKnot> c4;
+    load_block<64 * NQ * NQ>(msrc, nk * NQ * NQ, lane, m4);
+    load_block<64 * kDqddPerKnot>(csrc, nk * kDqddPerKnot, lane, c4);
     __builtin_amdgcn_sched_barrier(0);
-    copy_record_block<true>(rec, dqdd + prev * kDqddPerKnot, prev_words, lane);
+    copy_record_block<true, 64 * kDqddPerKnot>(rec, dqdd + prev * kDqddPerKnot, prev_words, lane);
     __builtin_amdgcn_sched_barrier(0);
     wave_lds_sync();
-    if (whole) put_block<64 * NQ * NQ>(m4, lane, rec);
-    else for (int e = lane; e < nk * NQ * NQ; e += 64) rec[e] = msrc[e];
+    put_block<64 * NQ * NQ>(m4, nk * NQ * NQ, lane, rec);
     wave_lds_sync();
     // lanes past the last knot read what the block holds and store nothing that is copied out
     float Mi[NQ][NQ];
@@ -606,8 +581,7 @@ __global__ __launch_bounds__(kBlock, 2) void finish_kernel(long n, const float* 
       });
     });
     wave_lds_sync();
-    if (whole) put_block<64 * kDqddPerKnot>(c4, lane, rec);
-    else for (int e = lane; e < nk * kDqddPerKnot; e += 64) rec[e] = csrc[e];
+    put_block<64 * kDqddPerKnot>(c4, nk * kDqddPerKnot, lane, rec);
     wave_lds_sync();
     InFinishRegs i{Mi, rec + kDqddPerKnot * lane};
     OutFinish o{rec + kDqddPerKnot * lane};
@@ -616,7 +590,7 @@ __global__ __launch_bounds__(kBlock, 2) void finish_kernel(long n, const float* 
     prev = k0;
     prev_words = nk * kDqddPerKnot;
   }
-  copy_record_block<true>(rec, dqdd + prev * kDqddPerKnot, prev_words, lane);
+  copy_record_block<true, 64 * kDqddPerKnot>(rec, dqdd + prev * kDqddPerKnot, prev_words, lane);
 }
 
 }  // namespace rbd
