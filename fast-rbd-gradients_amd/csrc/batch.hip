@@ -7,6 +7,7 @@
 #include <mutex>
 #include <new>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "batch_kernels.hpp"
@@ -27,10 +28,13 @@ struct rbd_batch {
   // counters of the last partial round (device memory, zero between launches)
   unsigned long long* d_tail = nullptr;
   size_t upload_bytes = 0;            // header + descriptors
-  // pinned host staging ring for the descriptor upload
+  // pinned, mapped host staging ring for the descriptors
   static constexpr int kRing = 4;
   char* h_stage[kRing] = {};
-  hipEvent_t staged[kRing] = {};
+  char* dh_stage[kRing] = {};         // their device addresses
+  hipEvent_t staged[kRing] = {};      // a slot's copy has read it, or
+  uint64_t read_seq[kRing] = {};      // the word in the slot that its staging kernel sets (0: none pending)
+  uint64_t next_seq = 0;
   int ring = 0;
   // persistent grid per shape, and the captured graphs per (shape, small
   // batch): index 2 * shape + small
@@ -58,6 +62,7 @@ namespace {
 size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 
 constexpr size_t kHeaderBytes = 256;   // the header's slot before the descriptors
+constexpr size_t kReadWord = 128;      // in it, the word that says the slot has been read
 constexpr int64_t kMaxBatchChunks = (int64_t(1) << 31) - 1;   // the kernels index chunks with int
 
 // Where a launch finds its queue: header and descriptors (the batch's own, or
@@ -69,6 +74,7 @@ struct Queue {
   const rbd::ArgBatch* args = nullptr;   // a small batch in the kernel arguments instead
   int64_t chunks = 0;                     // the batch's chunk total when known: no more waves than chunks
   rbd::Completion done{nullptr, 0};       // completion word, if the caller polls one
+  bool planned = false;                   // the prefix sum is already being made on the stream
 };
 
 // the batch's own header and descriptors, uploaded per launch
@@ -146,16 +152,15 @@ void launch_persistent(rbd_batch* b, const Queue& q, int wpg, hipStream_t s) {
 }
 
 // The persistent grids: as many waves as a CU keeps resident -- with one lane
-// per knot 6 (the 26,880-byte record blocks fill the LDS) with FP32 columns,
-// 4 (one per SIMD) with FP64 columns; with 16-lane groups two per SIMD with
-// FP32 columns, one with FP64 columns; two-wave workgroups at 256 registers,
+// per knot and with 16-lane groups two per SIMD with FP32 columns, one with
+// FP64 columns; two-wave workgroups at 256 registers,
 // one wave per SIMD; the L-lane groups one wave per SIMD, whatever their
 // workgroup size.
 void set_default_grid(rbd_batch* b) {
   const rbd_context* ctx = b->ctx;
   const bool fp32_columns = ctx->precision == RBD_PREC_FP32 || ctx->precision == RBD_PREC_FP64_PIVOT ||
                             ctx->precision == RBD_PREC_FP32_HW_TRIG;
-  b->grid[0] = unsigned(ctx->compute_units * (fp32_columns ? 6 : 4));
+  b->grid[0] = unsigned(ctx->compute_units * (fp32_columns ? 8 : 4));
   b->grid[1] = unsigned(ctx->compute_units * 4 * (fp32_columns ? 2 : 1));
   b->grid[2] = unsigned(ctx->compute_units * 2);
   for (int m = 3; m < rbd_batch::kMappings; ++m) b->grid[m] = unsigned(ctx->compute_units * 4);
@@ -222,7 +227,7 @@ hipError_t replay_small(rbd_batch* b, const rbd_traj* trajs, int n_traj, const r
 
 template <class P>
 hipError_t launch_batch_p(rbd_batch* b, const Queue& q, Shape sh, bool small, hipStream_t s) {
-  if (!small)
+  if (!small && !q.planned)
     hipLaunchKernelGGL(rbd::batch_plan_kernel, dim3(1), dim3(rbd::kPlanThreads), 0, s, q.descs, q.hdr, q.prefix);
   const int lanes = sh.lanes;
   const int wpg = is_group_lanes(lanes) && valid_wpg(sh.wpg) ? sh.wpg : 1;
@@ -268,6 +273,31 @@ long stage(char* dst, const rbd_traj* trajs, int n_traj, int lanes) {
   h->chunk_knots = is_group_lanes(lanes) ? 1 : int(chunk_knots(lanes));
   h->total_chunks = total;
   return total;
+}
+
+// The prefix sum the plan kernel would make, behind the staged descriptors
+void stage_prefix(char* dst, int n_traj) {
+  const rbd::BatchHeader* h = reinterpret_cast<const rbd::BatchHeader*>(dst);
+  const rbd::TrajDesc* d = reinterpret_cast<const rbd::TrajDesc*>(dst + kHeaderBytes);
+  long* p = reinterpret_cast<long*>(dst + batch_stage_bytes(n_traj));
+  long run = 0;
+  for (int t = 0; t < n_traj; ++t) {
+    p[t] = run;
+    run += (d[t].n + h->chunk_knots - 1) / h->chunk_knots;
+  }
+  p[n_traj] = run;
+}
+
+uint64_t* read_word(char* slot) { return reinterpret_cast<uint64_t*>(slot + kReadWord); }
+
+// Until the last batch staged in slot r has been read out of it.
+hipError_t wait_slot(rbd_batch* b, int r) {
+  const uint64_t seq = b->read_seq[r];
+  if (seq == 0) return hipEventSynchronize(b->staged[r]);
+  for (int spins = 0; __atomic_load_n(read_word(b->h_stage[r]), __ATOMIC_ACQUIRE) != seq; ++spins)
+    if (spins > (1 << 12)) std::this_thread::yield();       // the stream is four batches behind
+  b->read_seq[r] = 0;
+  return hipSuccess;
 }
 
 int graph_index(Shape sh, bool small) { return 2 * mapping_of(sh) + (small ? 1 : 0); }
@@ -356,8 +386,8 @@ rbd_status rbd_batch_create(rbd_context* ctx, int max_trajectories, rbd_batch** 
   static_assert(sizeof(rbd::BatchHeader) <= kHeaderBytes, "header slot");
   const size_t hdr = kHeaderBytes;
   const size_t desc = align_up(sizeof(rbd::TrajDesc) * size_t(max_trajectories), 256);
-  const size_t pre = sizeof(long) * (size_t(max_trajectories) + 1);
-  b->upload_bytes = hdr + sizeof(rbd::TrajDesc) * size_t(max_trajectories);
+  const size_t pre = align_up(sizeof(long) * (size_t(max_trajectories) + 1), 16);
+  b->upload_bytes = hdr + sizeof(rbd::TrajDesc) * size_t(max_trajectories) + pre;
   hipError_t e = hipMalloc(&b->d_mem, hdr + desc + pre);
   if (e != hipSuccess) { delete b; return fail(RBD_ERR_OUT_OF_MEMORY, "hipMalloc (batch)"); }
   b->d_hdr = reinterpret_cast<rbd::BatchHeader*>(b->d_mem);
@@ -374,6 +404,8 @@ rbd_status rbd_batch_create(rbd_context* ctx, int max_trajectories, rbd_batch** 
   }
   for (int i = 0; i < rbd_batch::kRing && e == hipSuccess; ++i) {
     e = hipHostMalloc(reinterpret_cast<void**>(&b->h_stage[i]), b->upload_bytes, hipHostMallocDefault);
+    if (e == hipSuccess) *read_word(b->h_stage[i]) = 0;
+    if (e == hipSuccess) e = hipHostGetDevicePointer(reinterpret_cast<void**>(&b->dh_stage[i]), b->h_stage[i], 0);
     if (e == hipSuccess) e = hipEventCreateWithFlags(&b->staged[i], hipEventDisableTiming);
   }
   if (e != hipSuccess) {
@@ -398,7 +430,8 @@ rbd_status rbd_batch_destroy(rbd_batch* b) {
     if (b->graph[gi]) (void)hipGraphDestroy(b->graph[gi]);
   }
   for (int i = 0; i < rbd_batch::kRing; ++i) {
-    if (b->staged[i]) { (void)hipEventSynchronize(b->staged[i]); (void)hipEventDestroy(b->staged[i]); }
+    if (b->h_stage[i] && b->staged[i]) (void)wait_slot(b, i);
+    if (b->staged[i]) (void)hipEventDestroy(b->staged[i]);
     if (b->h_stage[i]) (void)hipHostFree(b->h_stage[i]);
   }
   if (b->d_mem) (void)hipFree(b->d_mem);
@@ -477,12 +510,38 @@ rbd_status rbdi::batch_run(rbd_batch* b, const rbd_traj* trajs, int n_traj, int 
     if (le != hipSuccess) return hip_fail(le, "batch kernel launch");
     return RBD_OK;
   }
-  // stage header + descriptors in pinned memory, copy to the device on `stream`
+  // stage header and descriptors in pinned memory, from where a kernel or a
+  // copy on `stream` takes them; a stream under capture records the copy, since
+  // its kernel would set the slot's word only when the graph runs
   const int r = b->ring;
   b->ring = (r + 1) % rbd_batch::kRing;
-  hipError_t e = hipEventSynchronize(b->staged[r]);     // previous copy out of this slot is done
+  hipError_t e = wait_slot(b, r);     // the previous batch has been read out of this slot
   if (e != hipSuccess) return hip_fail(e, "staging wait");
   const int64_t chunks = stage(b->h_stage[r], trajs, n_traj, lanes);
+  hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+  if (!use_graph && n_traj <= rbd::kStageTrajectories) {
+    e = hipStreamIsCapturing(st, &capturing);
+    if (e != hipSuccess) return hip_fail(e, "stream status");
+  }
+  if (!use_graph && n_traj <= rbd::kStageTrajectories && capturing == hipStreamCaptureStatusNone) {
+    stage_prefix(b->h_stage[r], n_traj);
+    char* d_slot = b->dh_stage[r];
+    const uint64_t seq = ++b->next_seq;
+    hipLaunchKernelGGL(rbd::batch_stage_kernel, dim3(1), dim3(rbd::kPlanThreads), 0, st,
+                       reinterpret_cast<const rbd::v4i*>(d_slot + kHeaderBytes),
+                       *reinterpret_cast<const rbd::BatchHeader*>(b->h_stage[r]),
+                       reinterpret_cast<rbd::v4i*>(b->d_desc), b->d_hdr, reinterpret_cast<rbd::v4i*>(b->d_prefix),
+                       reinterpret_cast<unsigned long long*>(d_slot + kReadWord), (unsigned long long)seq);
+    e = hipGetLastError();
+    if (e != hipSuccess) return hip_fail(e, "batch staging kernel");
+    b->read_seq[r] = seq;
+    Queue q = own_queue(b);
+    q.chunks = chunks;
+    q.planned = true;
+    e = launch_batch(b, q, sh, small, st);
+    if (e != hipSuccess) return hip_fail(e, "batch kernel launch");
+    return RBD_OK;
+  }
   e = hipMemcpyAsync(b->d_mem, b->h_stage[r], batch_stage_bytes(n_traj), hipMemcpyHostToDevice, st);
   if (e == hipSuccess) e = hipEventRecord(b->staged[r], st);
   if (e != hipSuccess) return hip_fail(e, "descriptor upload");

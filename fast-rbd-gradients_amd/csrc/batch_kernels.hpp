@@ -39,6 +39,8 @@
 
 namespace rbd {
 
+typedef int v4i __attribute__((ext_vector_type(4)));
+
 struct TrajDesc {
   const float* in;   // n x 21 (AoS)
   float* out;        // n x 105 (AoS)
@@ -110,9 +112,60 @@ __global__ __launch_bounds__(kPlanThreads) void batch_plan_kernel(const TrajDesc
   if (threadIdx.x == kPlanThreads - 1) prefix[n] = partial[kPlanThreads - 1];
 }
 
+// Descriptors and prefix sum of a batch of up to kStageTrajectories
+// trajectories, from the pinned host block they were staged in (16-byte pieces:
+// two per trajectory, then the prefix sum two to a piece) to the batch's device
+// memory.  One block with every load in flight at once meets the bus's latency
+// once; it takes the place of a copy, an event and the plan kernel, whose scan
+// the host does while it writes the list (a call in a stream of calls, with
+// search_prefix below: 80 trajectories 20.9 -> 12.4 us, 1,024 36.3 -> 14.6,
+// 4,096 80.6 -> 34.9).  kStageTrajectories is what the threads hold at 11
+// pieces each; a longer list is copied (4,097: 61.4).  *done = seq tells the
+// host that the block has been read: every load has returned before the
+// barrier, so the store needs no release.
+constexpr int kStageTrajectories = 4096;
+__global__ __launch_bounds__(kPlanThreads) void batch_stage_kernel(const v4i* __restrict__ staged, BatchHeader h,
+                                                                   v4i* __restrict__ descs,
+                                                                   BatchHeader* __restrict__ hdr,
+                                                                   v4i* __restrict__ prefix,
+                                                                   unsigned long long* done, unsigned long long seq) {
+  const int t = int(threadIdx.x);
+  const int list = 2 * h.n_traj, pieces = list + (h.n_traj + 2) / 2;
+  constexpr int kEach = (2 * kStageTrajectories + (kStageTrajectories + 2) / 2 + kPlanThreads - 1) / kPlanThreads;
+  v4i x[kEach];
+  static_for<0, kEach>([&](auto Ec) {
+    constexpr int e = decltype(Ec)::value;
+    if (t + e * kPlanThreads < pieces) x[e] = staged[t + e * kPlanThreads];
+  });
+  static_for<0, kEach>([&](auto Ec) {
+    constexpr int e = decltype(Ec)::value;
+    const int i = t + e * kPlanThreads;
+    if (i < pieces) *(i < list ? descs + i : prefix + (i - list)) = x[e];
+  });
+  if (t == 0) *hdr = h;
+  __syncthreads();
+  if (t == 0) __hip_atomic_store(done, seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// The largest t below n with prefix[t] <= key (prefix[0] <= key), by the whole
+// wave: 64 places at a time, so two dependent loads for up to 4,096
+// trajectories where halving takes up to 12.
+__device__ inline int search_prefix(const long* prefix, int n, long key, int lane) {
+  int lo = 0, len = n;
+  while (len > 1) {
+    const int step = (len + 63) / 64;
+    const int at = lane * step;
+    const bool below = at < len && prefix[lo + at] <= key;
+    const int skip = (__popcll(__ballot(below)) - 1) * step;     // lane 0's place is at or below
+    lo += skip;
+    len = min(step, len - skip);
+  }
+  return lo;
+}
+
 // The trajectory t of chunk c and t's first chunk.  SMALL: the counts are
 // scanned in the calling wave, one trajectory per lane (every lane of the wave
-// takes part); otherwise a binary search of the plan kernel's prefix sum.
+// takes part); otherwise a search of the prefix sum by the whole wave.
 template <bool SMALL>
 __device__ inline void locate_chunk(const TrajDesc* descs, const long* prefix, int n_traj, int chunk, int c,
                                     int lane, int& t, int& first) {
@@ -127,13 +180,8 @@ __device__ inline void locate_chunk(const TrajDesc* descs, const long* prefix, i
     first = __shfl(v, t > 0 ? t - 1 : 0, 64);
     if (t == 0) first = 0;
   } else {
-    int lo = 0, hi = n_traj;               // prefix[lo] <= c < prefix[hi]
-    while (hi - lo > 1) {
-      const int mid = (lo + hi) >> 1;
-      if (prefix[mid] <= c) lo = mid; else hi = mid;
-    }
-    t = lo;
-    first = int(prefix[lo]);
+    t = search_prefix(prefix, n_traj, c, lane);
+    first = int(prefix[t]);
   }
 }
 
@@ -235,9 +283,9 @@ __global__ __launch_bounds__(64, kWavesPerSimd<P>) void batch_persistent_kernel(
   // (the chunk's inputs, 336 contiguous bytes, are read the same way into LDS
   // first: a few whole-line reads instead of many small per-lane ones)
   // one lane per knot: the chunk's records (64 consecutive knots of one
-  // trajectory, one contiguous block) are assembled in LDS and copied out
-  // whole (copy_record_block, streaming stores), as the flat one-lane kernel does
-  __shared__ __align__(16) float rec_sh[chunk * kOutPerKnot];
+  // trajectory, one contiguous block) leave through LDS as the flat one-lane
+  // kernel's do (put_records)
+  __shared__ __align__(16) float rec_sh[LANES == 1 ? kRecordLds<P, kOutPerKnot> : chunk * kOutPerKnot];
   __shared__ float in_sh[LANES == 1 ? 1 : chunk * kInPerKnot];
   auto process = [&](int c) {
     int t, first;                           // trajectory of chunk c, and its first chunk
@@ -249,13 +297,10 @@ __global__ __launch_bounds__(64, kWavesPerSimd<P>) void batch_persistent_kernel(
       const int knots = int(d.n - k0 < chunk ? d.n - k0 : chunk);
       // lanes past the trajectory's end compute a copy of its last knot and store nothing
       InAoS i{d.in + kInPerKnot * (k < d.n ? k : d.n - 1)};
-      OutAoS o{rec_sh + kOutPerKnot * slot};
+      float r[kHoldOutputs<P> ? kOutPerKnot : 1];
+      OutAoS o{kHoldOutputs<P> ? r : rec_sh + kOutPerKnot * slot};
       fdgrad_knot<P>(i, o, opt);
-      wave_lds_sync();
-      // streaming stores, as the flat kernel's (whole lines; made visible by
-      // the kernel's end or the completion word's release like any other store)
-      copy_record_block<true>(rec_sh, d.out + kOutPerKnot * k0, knots * kOutPerKnot, lane);
-      wave_lds_sync();                      // read out before the next chunk overwrites it
+      put_records<P, kOutPerKnot>(r, rec_sh, d.out + kOutPerKnot * k0, knots, lane);
     } else {
       const int knots = int(d.n - k0 < chunk ? d.n - k0 : chunk);
       for (int e = lane; e < knots * kInPerKnot; e += 64) in_sh[e] = d.in[kInPerKnot * k0 + e];
@@ -281,9 +326,9 @@ __global__ __launch_bounds__(64, kWavesPerSimd<P>) void batch_persistent_kernel(
 // trajectories and no lane idles at a trajectory's end: the 9,014 knots of 64
 // trajectories of 8..256 knots are 1,002 chunks of 9 with L = 7.  Each lane
 // finds its own knot's trajectory: SMALL batches from a shuffle scan of the
-// (up to 64) lengths, searched per lane; larger ones by a binary search of the
-// plan kernel's knot prefix sum (header chunk_knots = 1) for the chunk's first
-// knot, from which each lane walks on.  Workgroups of 1, 2 or 4 waves
+// (up to 64) lengths, searched per lane; larger ones by the wave's search of the
+// knot prefix sum (header chunk_knots = 1) for the chunk's first knot, from
+// which each lane walks on.  Workgroups of 1, 2 or 4 waves
 // (blockDim.x = 64 x waves), each wave on its own: its own chunks and LDS
 // block.  Queue, descriptors in the arguments and completion word as in
 // batch_persistent_kernel.
@@ -340,13 +385,7 @@ __global__ __launch_bounds__(kMaxGroupWaves * 64, 1) void batch_group_kernel(
       first = __shfl(incl, t > 0 ? t - 1 : 0, 64);
       if (t == 0) first = 0;
     } else {
-      const long kk0 = long(c) * Gr::kSlots;    // the chunk's first knot: wave-uniform search
-      int lo = 0, hi = n_traj;                  // prefix[lo] <= kk0 < prefix[hi]
-      while (hi - lo > 1) {
-        const int mid = (lo + hi) >> 1;
-        if (prefix[mid] <= kk0) lo = mid; else hi = mid;
-      }
-      t = lo;
+      t = search_prefix(prefix, n_traj, long(c) * Gr::kSlots, lane);     // of the chunk's first knot
       while (t + 1 < n_traj && prefix[t + 1] <= kk) ++t;
       first = prefix[t];
     }

@@ -360,8 +360,8 @@ rbd_status rbd_fdgrad_batched_f32(rbd_batch* b, const rbd_traj* trajs, int n_tra
 rbd_status rbd_fdgrad_batched_noalloc_f32(rbd_context* ctx, const rbd_traj* trajs, int n_traj, rbd_stream_t stream);
 
 /* Persistent grid size (waves) per mapping, lanes_per_knot 1, 4, 7, 8 or 16
- * (default: the waves the device's SIMDs keep resident: per CU 6 for one lane
- * and 8 for 16 lanes with FP32 columns, 4 for either with FP64 columns, 4 for
+ * (default: the waves the device's SIMDs keep resident: per CU 8 for one lane
+ * and for 16 lanes with FP32 columns, 4 for either with FP64 columns, 4 for
  * 4, 7 and 8 lanes in every workgroup size; the two-wave mapping runs 2
  * workgroups of two waves per CU).  The grid of the 4-, 7- and 8-lane groups
  * is set for all three of their workgroup sizes at once. */
