@@ -185,7 +185,13 @@ inline Shape shape_for(const rbd_context* ctx, int64_t n, bool full_path = false
     if (full_path && n <= ctx->two_wave_threshold.load(std::memory_order_relaxed)) return Shape{kTwoWaveLanes, 1};
     return Shape{n <= ctx->group_threshold.load(std::memory_order_relaxed) ? rbd::kLanesPerKnotGroup : 1, 1};
   }
-  if (!full_path && l != 1) return Shape{rbd::kLanesPerKnotGroup, 1};
+  if (!full_path && l != 1) {
+    // 16-lane groups hold 4 knots per wave and two waves per SIMD: up to 8
+    // knots per SIMD (8,192) they run in one round (8.8 us against 10.3 with
+    // one lane at 8,192 knots), beyond that in two (13.2 against 10.4 at 9,216)
+    const bool chosen = ctx->lanes_per_knot == 0;
+    return Shape{chosen && n > int64_t(32) * ctx->compute_units ? 1 : rbd::kLanesPerKnotGroup, 1};
+  }
   return Shape{l, wpg_for(ctx, ctx->tuned, l, n)};
 }
 inline int lanes_for(const rbd_context* ctx, int64_t n, bool full_path = false) {
