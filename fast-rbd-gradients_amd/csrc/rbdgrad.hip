@@ -73,17 +73,23 @@ __global__ __launch_bounds__(kBlock, kWavesPerSimd<P>) void fdgrad_aos_kernel(lo
       });
 }
 
-// Structure-of-arrays output of the one-lane kernel with streaming
-// (non-temporal) stores: each store writes one output row for the wave's 64
-// consecutive knots, 256 contiguous bytes, written once.  At 2^20 knots the
-// kernel measured 162 against 186 us with plain stores, whose write-allocated
-// lines kept the waves waiting.  The last column computed (d/dqd column 0;
-// the columns come from the tip's to the base's) is kept in `last` instead of
-// stored: the kernel stores it after the next knot's input loads have issued.
-struct OutSoAStream {
+// Structure-of-arrays output of the one-lane kernel: each store writes one
+// output row for the wave's 64 consecutive knots, 256 contiguous bytes, written
+// once.  NT: streaming (non-temporal) stores, for rows that start on a line
+// (aligned_rows): at 2^20 knots 102 us against 122 with plain stores, whose
+// write-allocated lines keep the waves waiting.  Other rows share the line at
+// each end of a wave's 256 bytes with the neighbouring wave, and streamed out
+// in two parts such a line costs the memory side a read and two writes; plain
+// stores leave it in the L2 until the neighbour has written its part (1,000,003
+// knots in rows of as many: 171 us against 222; 300,007: 36 against 65).  The
+// last column computed (d/dqd column 0; the columns come from the tip's to the
+// base's) is kept in `last` instead of stored: the kernel stores it after the
+// next knot's input loads have issued.
+template <bool NT>
+struct OutSoARows {
   float* p; long ld;
   float* last;
-  __device__ void st(long row, float x) const { put<true>(p + row * ld, x); }
+  __device__ void st(long row, float x) const { put<NT>(p + row * ld, x); }
   __device__ void qdd(int i, float x) const { st(i, x); }
   __device__ void dq(int r, int c, float x) const { st(NQ + NQ * c + r, x); }
   __device__ void dqd(int r, int c, float x) const {
@@ -92,32 +98,39 @@ struct OutSoAStream {
   }
 };
 
+constexpr int kXcds = 8;
+
 // One lane per knot, structure of arrays.  As in the AoS kernel, each loop
 // iteration issues its knot's input loads before any store: here the previous
 // knot's last column, so the wait for the loads covers only stores issued a
 // column's work earlier, which have retired.  At 2^20 knots: 156.0-157.0
 // against 162.0-162.2 us with the last column stored at the end of its own
-// iteration, bitwise the same results.
-template <class P>
+// iteration, bitwise the same results.  Workgroups are dealt to the 8 XCDs in
+// turn; each XCD's take one run of neighbouring knots, so that lines shared by
+// two waves are shared within one L2 (1,000,003 knots, plain stores: 171 us
+// against 200; 131,072 knots, streaming stores: 15.4 against 17.1).
+template <class P, bool NT>
 __global__ __launch_bounds__(kBlock, kWavesPerSimd<P>) void fdgrad_soa_kernel(long n, const float* __restrict__ in, long ld_in,
                                                             float* __restrict__ out, long ld_out, Options opt) {
   constexpr int kLastRow = NQ + NQ * NQ;     // d/dqd column 0
   const long stride = long(gridDim.x) * blockDim.x;
   float last[NQ];
   long prev = -1;
-  for (long k = long(blockIdx.x) * blockDim.x + threadIdx.x; k < n; k += stride) {
+  const int xcd = int(blockIdx.x) % kXcds, per_xcd = int(gridDim.x) / kXcds, more = int(gridDim.x) % kXcds;
+  const int place = xcd * per_xcd + min(xcd, more) + int(blockIdx.x) / kXcds;
+  for (long k = long(place) * blockDim.x + threadIdx.x; k < n; k += stride) {
     InRegs i;
     for (int j = 0; j < kInPerKnot; ++j) i.x[j] = in[j * ld_in + k];
     __builtin_amdgcn_sched_barrier(0);
     if (prev >= 0)
-      for (int r = 0; r < NQ; ++r) put<true>(out + (kLastRow + r) * ld_out + prev, last[r]);
+      for (int r = 0; r < NQ; ++r) put<NT>(out + (kLastRow + r) * ld_out + prev, last[r]);
     __builtin_amdgcn_sched_barrier(0);
-    OutSoAStream o{out + k, ld_out, last};
+    OutSoARows<NT> o{out + k, ld_out, last};
     fdgrad_knot<P>(i, o, opt);
     prev = k;
   }
   if (prev >= 0)
-    for (int r = 0; r < NQ; ++r) put<true>(out + (kLastRow + r) * ld_out + prev, last[r]);
+    for (int r = 0; r < NQ; ++r) put<NT>(out + (kLastRow + r) * ld_out + prev, last[r]);
 }
 
 // Reference-compatible mode (qdd and Minv given), one lane per knot, records
@@ -656,6 +669,12 @@ hipError_t one_lane_grid(int cus, dim3* grid) {
   return hipSuccess;
 }
 
+// Whether every output row of a structure-of-arrays call starts on a 128-byte
+// line (fdgrad_soa_kernel).
+bool aligned_rows(const FlatCall& c) {
+  return reinterpret_cast<uintptr_t>(c.out) % 128 == 0 && c.ld_out % 32 == 0;
+}
+
 template <class P>
 hipError_t launch_flat_p(const FlatCall& c) {
   dim3 grid(grid_for(c.n, c.lanes)), block(kBlock);
@@ -664,7 +683,10 @@ hipError_t launch_flat_p(const FlatCall& c) {
     hipError_t e = hipSuccess;
     switch (c.layout) {
       case Layout::AoS: e = one_lane_grid<rbd::fdgrad_aos_kernel<P>>(c.simds / 4, &grid); break;   // 4 SIMDs per CU
-      case Layout::SoA: e = one_lane_grid<rbd::fdgrad_soa_kernel<P>>(c.simds / 4, &grid); break;
+      case Layout::SoA:
+        e = aligned_rows(c) ? one_lane_grid<rbd::fdgrad_soa_kernel<P, true>>(c.simds / 4, &grid)
+                            : one_lane_grid<rbd::fdgrad_soa_kernel<P, false>>(c.simds / 4, &grid);
+        break;
       case Layout::Ref: e = one_lane_grid<rbd::fdgrad_refmode_kernel<P>>(c.simds / 4, &grid); break;
     }
     if (e != hipSuccess) return e;
@@ -673,8 +695,12 @@ hipError_t launch_flat_p(const FlatCall& c) {
         hipLaunchKernelGGL(rbd::fdgrad_aos_kernel<P>, grid, block, 0, c.stream, n, c.in, c.out, c.opt);
         break;
       case Layout::SoA:
-        hipLaunchKernelGGL(rbd::fdgrad_soa_kernel<P>, grid, block, 0, c.stream, n, c.in, long(c.ld_in), c.out,
-                           long(c.ld_out), c.opt);
+        if (aligned_rows(c))
+          hipLaunchKernelGGL((rbd::fdgrad_soa_kernel<P, true>), grid, block, 0, c.stream, n, c.in, long(c.ld_in),
+                             c.out, long(c.ld_out), c.opt);
+        else
+          hipLaunchKernelGGL((rbd::fdgrad_soa_kernel<P, false>), grid, block, 0, c.stream, n, c.in, long(c.ld_in),
+                             c.out, long(c.ld_out), c.opt);
         break;
       case Layout::Ref:
         hipLaunchKernelGGL(rbd::fdgrad_refmode_kernel<P>, grid, block, 0, c.stream, n, c.in, c.out, c.opt);

@@ -1,9 +1,9 @@
 """GPU tests of rules that take a call to one path or another by its size:
 the mapping of entry points without kernels of their own for small lane groups
-(16-lane groups up to 8 knots per SIMD, one lane above), the whole-line load
-of external forces (sets in a row, 16-byte aligned, a full block of 64 knots),
-and how a batch's list of trajectories reaches the device (kernel arguments up
-to 64, one staging kernel up to 1,024, a copy and a plan kernel above)."""
+(16-lane groups up to 8 knots per SIMD, one lane above), streaming or plain
+stores of structure-of-arrays rows (rows that start on a line, or not) and how
+a batch's list of trajectories reaches the device (kernel arguments up to 64, one staging
+kernel up to 4,096, a copy and a plan kernel above)."""
 import ctypes
 
 import numpy as np
@@ -42,6 +42,30 @@ def test_mapping_without_small_groups(rbd, n, lanes):
         got.append(fext_call(rbd, ctx, x, f))
         ctx.close()
     np.testing.assert_array_equal(got[0], got[1])
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 511, 513, 640, 131201])
+def test_soa_row_alignment(rbd, n):
+    """Rows aligned or not: the array-of-structures result bit for bit, and
+    nothing written between the rows."""
+    x = common.knots(n, seed=740)
+    ctx = rbd.Context(lanes_per_knot=1)
+    d_in, d_out = rbd.DeviceBuffer.from_array(x), rbd.DeviceBuffer(n * 420)
+    ctx.fdgrad(n, d_in, d_out)
+    want = d_out.download((n, 105))
+    whole = (n + 31) // 32 * 32
+    for ld, offset in ((whole, 0), (whole, 64), (whole + 16, 0), (whole + 1, 0), (n, 4)):
+        print(f"soa n={n} ld={ld} offset={offset}", flush=True)
+        xt = np.zeros((21, ld), np.float32)
+        xt[:, :n] = x.T
+        d_x = rbd.DeviceBuffer.from_array(xt)
+        d_y = rbd.DeviceBuffer.from_array(np.full(105 * ld + 32, 7.5, np.float32))
+        ctx.fdgrad_soa(n, d_x, ld, At(d_y, offset), ld)
+        raw = d_y.download((105 * ld + 32,))
+        got = raw[offset // 4:offset // 4 + 105 * ld].reshape(105, ld)
+        np.testing.assert_array_equal(got[:, :n], want.T)
+        assert np.all(got[:, n:] == 7.5) and np.all(raw[:offset // 4] == 7.5) and np.all(raw[offset // 4 + 105 * ld:] == 7.5)
+    ctx.close()
 
 
 @pytest.mark.parametrize("lanes", [0, 1])
