@@ -1,24 +1,23 @@
 // Per-knot-point forward-dynamics gradient of the KUKA iiwa 14, register resident.
 //
 // One call computes, for one knot point, q, qd, u -> qdd, dqdd/dq, dqdd/dqd with
-// the reference's method (plancherb1/fast-rbd-gradients):
+// the reference's results (plancherb1/fast-rbd-gradients); the steps:
 //   1. sin/cos of q and the seven joint transforms  (dynamicsGradient.h:507-587)
-//   2. Minv by the articulated-body recursion         (minv.h:423-478)
+//   2. the articulated-body recursion: the mass matrix's factors, or Minv
+//      where it is an output or shared by lanes       (minv.h:423-478)
 //   3. RNEA with qdd = 0 -> bias c                    (dynamicsGradient.h:619-683)
 //   4. qdd = Minv (u - c)                             (dynamicsGradient.h:704)
 //   5. RNEA with qdd: v, a, f                         (dynamicsGradient.h:893-895)
-//   6. dtau/dq, dtau/dqd: forward sweep over links per column, backward sweep
+//   6. dtau/dq, dtau/dqd: from composite quantities in one lane, by a forward
+//      and a backward sweep over the links per column in a lane group
 //                                                     (dynamicsGradient.h:786-857)
 //   7. dqdd/d(q,qd) = -Minv dtau/d(q,qd)              (dynamicsGradient.h:921)
 // Every link index is a compile-time constant (static_for), so each joint's
 // transform, inertia and offset are folded into straight-line code: structural
 // zeros of E, r and I cost nothing when the file is compiled with
 // -fno-signed-zeros -ffinite-math-only (these let x*0 and x+0 fold away).
-// In one lane the thirteen columns of step 6 are unrolled at compile time, so
-// each column's sweep starts at its own link with its seed folded into the
-// code (a lane group instead gives each lane a run-time column of its own,
-// dtau_column_uniform); each output column -Minv dtau[:, c] is stored as soon
-// as it is known, so dtau never has to be held whole.
+// A lane group gives each lane run-time columns of its own
+// (dtau_column_uniform).
 //
 // The file is plain C++17 when RBD_HD is empty, so the same arithmetic is also
 // compiled for the host by the CPU test harness.
@@ -338,9 +337,29 @@ template <int K, int I, typename S>
 RBD_HD RBD_INLINE S fixed(const S* x) {
   return fma_s(kFixed<S, K, I, 0>, x[0], fma_s(kFixed<S, K, I, 1>, x[1], kFixed<S, K, I, 2> * x[2]));
 }
+// Entry (I, J) of E = Rz(q)^T F.  Where F is no signed permutation, a rotation
+// by E's entries (formed once per link and shared by all its rotations) takes 9
+// instructions and one by F, then Rz, 13.  Synthetic arm: 128 knots 6.35 -> 6.05
+// us, 2,500 knots 7.3 -> 6.7, 9,000 knots 10.5 -> 10.0; in one lane the entries
+// cost registers (216 bytes of spills; 20,000 knots 15.4 -> 14.9 us, 2^20 knots
+// 164 -> 173), and one form serves all mappings so that they round alike.
+template <int K, int I, int J, typename S>
+RBD_HD RBD_INLINE S rot_entry(const CS<S>& t) {
+  if constexpr (I == 0) return fma_s(t.c, kFixed<S, K, 0, J>, t.s * kFixed<S, K, 1, J>);
+  else if constexpr (I == 1) return fma_s(t.c, kFixed<S, K, 1, J>, -t.s * kFixed<S, K, 0, J>);
+  else return kFixed<S, K, 2, J>;
+}
 // y = E x
 template <int K, typename S>
 RBD_HD RBD_INLINE void to_child(const CS<S>& t, const S* x, S* y) {
+  if constexpr (!signed_permutation<K>()) {
+    const S x0 = x[0], x1 = x[1], x2 = x[2];
+    static_for<0, 3>([&](auto Ic) {
+      constexpr int i = decltype(Ic)::value;
+      y[i] = fma_s(rot_entry<K, i, 0>(t), x0, fma_s(rot_entry<K, i, 1>(t), x1, rot_entry<K, i, 2>(t) * x2));
+    });
+    return;
+  }
   const S w0 = fixed<K, 0>(x), w1 = fixed<K, 1>(x), w2 = fixed<K, 2>(x);
   y[0] = fma_s(t.s, w1, t.c * w0);
   y[1] = fma_s(-t.s, w0, t.c * w1);
@@ -349,6 +368,14 @@ RBD_HD RBD_INLINE void to_child(const CS<S>& t, const S* x, S* y) {
 // y = E^T x, and y = E^T x + z
 template <int K, typename S>
 RBD_HD RBD_INLINE void to_parent(const CS<S>& t, const S* x, S* y) {
+  if constexpr (!signed_permutation<K>()) {
+    const S x0 = x[0], x1 = x[1], x2 = x[2];
+    static_for<0, 3>([&](auto Jc) {
+      constexpr int j = decltype(Jc)::value;
+      y[j] = fma_s(rot_entry<K, 0, j>(t), x0, fma_s(rot_entry<K, 1, j>(t), x1, rot_entry<K, 2, j>(t) * x2));
+    });
+    return;
+  }
   const S w[3] = {fma_s(-t.s, x[1], t.c * x[0]), fma_s(t.s, x[0], t.c * x[1]), x[2]};
   const S y0 = fixed_t<K, 0>(w), y1 = fixed_t<K, 1>(w), y2 = fixed_t<K, 2>(w);
   y[0] = y0; y[1] = y1; y[2] = y2;
@@ -362,9 +389,12 @@ RBD_HD RBD_INLINE void to_parent_add(const CS<S>& t, const S* x, const S* z, S* 
     const S y0 = fixed_t<K, 0>(w), y1 = fixed_t<K, 1>(w), y2 = fixed_t<K, 2>(w);
     y[0] = y0; y[1] = y1; y[2] = y2;
   } else {
-    S w[3];
-    to_parent<K>(t, x, w);
-    y[0] = z[0] + w[0]; y[1] = z[1] + w[1]; y[2] = z[2] + w[2];
+    const S x0 = x[0], x1 = x[1], x2 = x[2];
+    static_for<0, 3>([&](auto Jc) {
+      constexpr int j = decltype(Jc)::value;
+      y[j] = fma_s(rot_entry<K, 0, j>(t), x0,
+                   fma_s(rot_entry<K, 1, j>(t), x1, fma_s(rot_entry<K, 2, j>(t), x2, z[j])));
+    });
   }
 }
 // y += r x f, r joint K's offset
@@ -490,9 +520,9 @@ using PrecFP64      = Precision<double, double, double, double>; // all FP64
 
 // Waves each SIMD keeps resident for the kernels of precision P.  With FP32
 // RNEA and columns a knot's state fits in 256 registers per lane, so two waves
-// share a SIMD and each hides the other's latency (1.44x the throughput of one
-// wave at 2^20 knots when measured); with FP64 columns it needs about 500 and
-// runs one.
+// share a SIMD: a wave issues at most one instruction every 4 cycles, so two
+// issue twice as many (and each hides the other's latency); with FP64 columns
+// it needs about 500 and runs one.
 template <class P>
 constexpr int kWavesPerSimd = (sizeof(typename P::Col) == 4 && sizeof(typename P::Rnea) == 4) ? 2 : 1;
 
