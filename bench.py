@@ -57,22 +57,21 @@ REL_TOL = 1e-4                # the accuracy bar: max relative error per output 
 LARGE = 1 << 20               # knots of the large batch
 # HBM bytes per launch measured with rocprofv3 --pmc FETCH_SIZE and WRITE_SIZE
 # (x2.000 and x1.000, the factors a device-to-device copy of known size gives;
-# KiB per dispatch): profiles/fdgrad_large_batch_2p20_soa_aos.md and
-# profiles/fdgrad_per_call_n128.md.  Keyed by (kernel, knots per launch);
+# KiB per dispatch): profiles/fdgrad_range_of_calls.md.  Keyed by (kernel, knots per launch);
 # other configurations report null.
 MEASURED_TRAFFIC_BYTES = {
-    ("fdgrad_two_wave_kernel<PrecFP32>", 128): int((176.0 * 2.000 + 53.0 * 1.000) * 1024),
-    ("fdgrad_soa_kernel<PrecFP32>", LARGE): int((41326.1 * 2.000 + 430108.3) * 1024),
-    ("fdgrad_aos_kernel<PrecFP32>", LARGE): int((43356.5 * 2.000 + 430334.7) * 1024),
+    ("fdgrad_two_wave_kernel<PrecFP32>", 128): int((170.5 * 2.000 + 53.0 * 1.000) * 1024),
+    ("fdgrad_soa_kernel<PrecFP32>", LARGE): int((41202.5 * 2.000 + 430174.0) * 1024),
+    ("fdgrad_aos_kernel<PrecFP32>", LARGE): int((43246.0 * 2.000 + 430192.9) * 1024),
 }
 # Executed work of the one-lane FP32 kernel per 64-knot block (one knot per
 # lane), from rocprofv3 --pmc SQ_INSTS_VALU and SQ_INSTS_VALU_FLOPS_FP32 at 2^20
-# knots (profiles/fdgrad_large_batch_2p20_soa_aos.md): VALU instructions, and
+# knots (profiles/fdgrad_range_of_calls.md): VALU instructions, and
 # FP32 FLOPs per knot (an FMA counts 2).  The algorithmic count above is the
 # reference method's, whose dense 6x6 inertia products include structural
 # zeros the kernel never computes, so its roofline fraction can pass 1.
-EXECUTED_VALU_PER_KNOT = 6599
-EXECUTED_FLOPS_PER_KNOT = 10900
+EXECUTED_VALU_PER_KNOT = 3600
+EXECUTED_FLOPS_PER_KNOT = 5590
 N_SET = (1, 10, 16, 32, 64, 128, 256)   # trajectory lengths of the reference's harness (time_GPU.cu:344-351)
 HARNESS = os.path.join(PKG, "harness", "time_gpu")
 

@@ -5,8 +5,8 @@
 // input bytes and its 420 output bytes, plus LDS exchanges inside a knot's
 // lane group:
 //   * one lane per knot (throughput): a wave computes 64 knots in lock step
-//     with uniform control flow (the derivative columns are unrolled at
-//     compile time, the same column in every lane);
+//     with uniform control flow (the derivative columns from composite
+//     quantities, the same in every lane);
 //   * one knot per group of 4, 7 or 8 lanes (group_mapping.hpp): every lane
 //     runs the shared steps and a share of the derivative columns;
 //   * one knot per 16-lane group: the shared steps, then one derivative column
