@@ -403,7 +403,10 @@ rbd_status rbd_batch_create(rbd_context* ctx, int max_trajectories, rbd_batch** 
     return fail(RBD_ERR_OUT_OF_MEMORY, "batch queue counters");
   }
   for (int i = 0; i < rbd_batch::kRing && e == hipSuccess; ++i) {
-    e = hipHostMalloc(reinterpret_cast<void**>(&b->h_stage[i]), b->upload_bytes, hipHostMallocDefault);
+    // coherent: the staging kernel reads a slot that the host has just rewritten
+    // and the host polls the word it sets
+    e = hipHostMalloc(reinterpret_cast<void**>(&b->h_stage[i]), b->upload_bytes,
+                      hipHostMallocMapped | hipHostMallocCoherent);
     if (e == hipSuccess) *read_word(b->h_stage[i]) = 0;
     if (e == hipSuccess) e = hipHostGetDevicePointer(reinterpret_cast<void**>(&b->dh_stage[i]), b->h_stage[i], 0);
     if (e == hipSuccess) e = hipEventCreateWithFlags(&b->staged[i], hipEventDisableTiming);
