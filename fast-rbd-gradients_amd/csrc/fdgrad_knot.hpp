@@ -1139,14 +1139,17 @@ RBD_HD RBD_INLINE void derivative_columns(const In& in, const CS<S>* t, const S 
         to_parent<u>(t[u], bs, bs);
         tq[j][k] = g[2];
         td[j][k] = gd[2];
-        if constexpr (j > 0) {
+        if constexpr (j > 0 || F_GIVEN) {
           S Dj[6], Pj[6];
           motion_pair(v[j], a[j], Dj, Pj);
           td[k][j] = fma_s(is[0], Dj[0], fma_s(is[1], Dj[1], fma_s(is[3], Dj[3], fma_s(is[4], Dj[4], S(2) * bs[2]))));
-          tq[k][j] = fma_s(is[0], Pj[0], fma_s(is[1], Pj[1], fma_s(is[2], Pj[2], fma_s(is[3], Pj[3],
-                     fma_s(is[4], Pj[4], fma_s(is[5], Pj[5], fma_s(bs[0], Dj[0], bs[1] * Dj[1])))))));
+          if constexpr (j > 0)
+            tq[k][j] = fma_s(is[0], Pj[0], fma_s(is[1], Pj[1], fma_s(is[2], Pj[2], fma_s(is[3], Pj[3],
+                       fma_s(is[4], Pj[4], fma_s(is[5], Pj[5], fma_s(bs[0], Dj[0], bs[1] * Dj[1])))))));
         } else {
-          td[k][0] = S(2) * bs[2];                                     // link 0 only turns: D_0 = 0
+          // link 0 only turns, D_0 = 0; where the velocities are given they may
+          // be those of an arm on a moving base
+          td[k][0] = S(2) * bs[2];
         }
       });
     }
