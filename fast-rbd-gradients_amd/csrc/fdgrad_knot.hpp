@@ -458,21 +458,53 @@ RBD_HD RBD_INLINE void add_force_cross(const S* x, const S* z, S* y) {
 
 // Symmetric 3x3 matrices are stored as xx, xy, xz, yy, yz, zz.
 RBD_HD constexpr int sym(int i, int j) { return (i == 0 || j == 0) ? i + j : i + j + 1; }
-// products of a joint's sin and cos: sin^2 q, sin 2q, cos 2q, sin(2q) / 2
-template <typename S> struct DoubleAngle { S ss, s2, c2, sc; };
+// products of a joint's sin and cos: cos^2 q, sin^2 q, sin 2q, cos 2q, sin(2q) / 2
+template <typename S> struct DoubleAngle { S cc, ss, s2, c2, sc; };
 template <typename S>
 RBD_HD RBD_INLINE DoubleAngle<S> double_angle(const CS<S>& t) {
   const S ss = t.s * t.s, sc = t.c * t.s;
-  return {ss, sc + sc, fma_s(S(-2), ss, S(1)), sc};
+  return {t.c * t.c, ss, sc + sc, fma_s(S(-2), ss, S(1)), sc};
 }
-// A = E^T A E.  The z rotation leaves the trace of the x-y block, so the block
-// takes 7 operations instead of the 14 of two one-sided rotations.
-template <int K, typename S>
+// A = E^T A E.  Where F is a signed permutation: the z rotation leaves the trace
+// of the x-y block, so the block takes 7 operations instead of the 14 of two
+// one-sided rotations.  SMALL_DIAGONAL: a diagonal entry may come out far below
+// the other (the articulated inertia about a slender link's axis, the pivot),
+// and as the difference of two large numbers it would keep their rounding
+// error: its terms are summed instead (3 operations more).  Error of dqdd/dq in
+// lane groups, FP32: 2.07e-7 against 2.14e-7 of its norm.  Other F: two
+// one-sided rotations by E's entries, which also take fewer instructions than
+// the z rotation and F on both sides (synthetic arm, dqdd/dq 4.37e-7 against
+// 4.58e-7; 104 instructions fewer in a factorisation).
+template <int K, bool SMALL_DIAGONAL, typename S>
 RBD_HD RBD_INLINE void sym_to_parent(const CS<S>& t, const DoubleAngle<S>& q, S A[6]) {
+  if constexpr (!signed_permutation<K>()) {
+    S Y[3][3];                                   // A E
+    static_for<0, 3>([&](auto Rc) {
+      constexpr int r = decltype(Rc)::value;
+      const S row[3] = {A[sym(r, 0)], A[sym(r, 1)], A[sym(r, 2)]};
+      to_parent<K>(t, row, Y[r]);
+    });
+    static_for<0, 3>([&](auto Jc) {
+      constexpr int j = decltype(Jc)::value;
+      const S col[3] = {Y[0][j], Y[1][j], Y[2][j]};
+      S y[3];
+      to_parent<K>(t, col, y);
+      for (int i = 0; i <= j; ++i) A[sym(i, j)] = y[i];
+    });
+    return;
+  }
   const S d = A[3] - A[0];
-  const S e = fma_s(-q.s2, A[1], q.ss * d);
-  const S B[6] = {A[0] + e, fma_s(-q.sc, d, q.c2 * A[1]), fma_s(-t.s, A[4], t.c * A[2]),
-                  A[3] - e, fma_s(t.s, A[2], t.c * A[4]), A[5]};
+  S b0, b3;
+  if constexpr (SMALL_DIAGONAL) {
+    b0 = fma_s(-q.s2, A[1], fma_s(q.ss, A[3], q.cc * A[0]));
+    b3 = fma_s(q.s2, A[1], fma_s(q.ss, A[0], q.cc * A[3]));
+  } else {
+    const S e = fma_s(-q.s2, A[1], q.ss * d);
+    b0 = A[0] + e;
+    b3 = A[3] - e;
+  }
+  const S B[6] = {b0, fma_s(-q.sc, d, q.c2 * A[1]), fma_s(-t.s, A[4], t.c * A[2]),
+                  b3, fma_s(t.s, A[2], t.c * A[4]), A[5]};
   static_for<0, 3>([&](auto Ic) {
     constexpr int i = decltype(Ic)::value;
     S col[3];                                    // column i of B F
@@ -589,9 +621,9 @@ RBD_HD RBD_INLINE void move_articulated(const CS<S>& t, const S a[3], const S c[
                                         S TR[3][3], S BR[6]) {
   const DoubleAngle<S> q = double_angle(t);
   TL[0] = a[0]; TL[1] = a[1]; TL[3] = a[2]; TL[2] = S(0); TL[4] = S(0); TL[5] = S(0);
-  sym_to_parent<K>(t, q, TL);
+  sym_to_parent<K, true>(t, q, TL);
   for (int i = 0; i < 6; ++i) BR[i] = n[i];
-  sym_to_parent<K>(t, q, BR);
+  sym_to_parent<K, true>(t, q, BR);
   S r0[3], r1[3], C[3][3];                       // C E, then E^T (C E)
   to_parent<K>(t, c[0], r0);
   to_parent<K>(t, c[1], r1);
@@ -687,7 +719,14 @@ RBD_HD RBD_INLINE void mass_factors(const CS<S>* t, MassFactors<S>& f) {
   });
 }
 
-// x = M^-1 x (NEG: negated)
+// x = M^-1 x, or -M^-1 x (NEG, a derivative column).  The back substitution of a
+// solve sums its products first and takes them from y_k / D_k in one
+// multiply-add, whose product is not rounded: y_k / D_k is often far above the
+// result, and with the sum started from it every step rounds at its size
+// (error of qdd in FP32 7.1e-8 of its norm, so 4.9e-8).  A derivative column is
+// started from it all the same: it gains little (dqdd/dq 2.03e-7, so 1.98e-7),
+// and with the sum beside y_k the one-lane kernels are a register short (external
+// forces at 150,001 knots 24.6 us, so 26.0).
 template <bool NEG, typename S, typename SX>
 RBD_HD RBD_INLINE void mass_solve(const MassFactors<S>& f, SX x[NQ]) {
   static_for_down<NQ, 1>([&](auto Kc) {
@@ -697,20 +736,35 @@ RBD_HD RBD_INLINE void mass_solve(const MassFactors<S>& f, SX x[NQ]) {
       x[j] = fma_s(-SX(f.L[k][j]), x[k], x[j]);
     });
   });
-  for (int k = 0; k < NQ; ++k) x[k] = (NEG ? -x[k] : x[k]) * SX(f.dinv[k]);
-  static_for<1, NQ>([&](auto Kc) {
-    constexpr int k = decltype(Kc)::value;
-    static_for<0, k>([&](auto Jc) {
-      constexpr int j = decltype(Jc)::value;
-      x[k] = fma_s(-SX(f.L[k][j]), x[j], x[k]);
+  if constexpr (NEG) {
+    for (int k = 0; k < NQ; ++k) x[k] = -x[k] * SX(f.dinv[k]);
+    static_for<1, NQ>([&](auto Kc) {
+      constexpr int k = decltype(Kc)::value;
+      static_for<0, k>([&](auto Jc) {
+        constexpr int j = decltype(Jc)::value;
+        x[k] = fma_s(-SX(f.L[k][j]), x[j], x[k]);
+      });
     });
-  });
+  } else {
+    x[0] *= SX(f.dinv[0]);
+    static_for<1, NQ>([&](auto Kc) {
+      constexpr int k = decltype(Kc)::value;
+      SX sum = SX(f.L[k][0]) * x[0];
+      static_for<1, k>([&](auto Jc) {
+        constexpr int j = decltype(Jc)::value;
+        sum = fma_s(SX(f.L[k][j]), x[j], sum);
+      });
+      x[k] = fma_s(x[k], SX(f.dinv[k]), -sum);
+    });
+  }
 }
 
 // Column j of Minv from the factors: col[k] = Minv[k][j] for k <= j (the
 // entries below are formed too far only to k = j when J is a constant, and
 // left unspecified).  The forward sums of links k > j are exactly zero, so the
-// run-time j of the lane groups gives bitwise the entries of a constant j.
+// run-time j of the lane groups gives bitwise the entries of a constant j.  The
+// products are summed first, as in mass_solve (error of Minv in FP32 5.6e-8 of
+// its norm, so 3.8e-8).
 template <int J, typename S>
 RBD_HD RBD_INLINE void minv_column(const MassFactors<S>& f, int j, S col[NQ]) {
   constexpr int top = J < 0 ? NQ : J + 1;        // rows to form
@@ -726,12 +780,16 @@ RBD_HD RBD_INLINE void minv_column(const MassFactors<S>& f, int j, S col[NQ]) {
   });
   static_for<0, top>([&](auto Kc) {
     constexpr int k = decltype(Kc)::value;
-    S acc = y[k] * f.dinv[k];
-    static_for<0, k>([&](auto Ic) {
-      constexpr int i = decltype(Ic)::value;
-      acc = fma_s(-f.L[k][i], col[i], acc);
-    });
-    col[k] = acc;
+    if constexpr (k == 0) {
+      col[0] = y[0] * f.dinv[0];
+    } else {
+      S sum = f.L[k][0] * col[0];
+      static_for<1, k>([&](auto Ic) {
+        constexpr int i = decltype(Ic)::value;
+        sum = fma_s(f.L[k][i], col[i], sum);
+      });
+      col[k] = fma_s(y[k], f.dinv[k], -sum);
+    }
   });
 }
 
@@ -1069,7 +1127,7 @@ RBD_HD RBD_INLINE void composite_step(const In& in, const CS<S>* t, const S* v, 
     const DoubleAngle<S> q = double_angle(t[u]);
     // inertia about the new origin: i + 2 (r.h) 1 - h r^T - r h^T + m (r.r 1 - r r^T), then the link's own
     to_parent<u>(t[u], c.h, c.h);
-    sym_to_parent<u>(t[u], q, c.i);
+    sym_to_parent<u, false>(t[u], q, c.i);
     add_sym_outer<S>(S(1), S(r[0]), S(r[1]), S(r[2]), c.h, c.i);
     static_for<0, 3>([&](auto Ic) {
       constexpr int i = decltype(Ic)::value;
@@ -1083,7 +1141,7 @@ RBD_HD RBD_INLINE void composite_step(const In& in, const CS<S>* t, const S* v, 
     });
     // Bs likewise with the momentum p in h's place; the momentum moves as a force
     to_parent<u>(t[u], c.p, c.p);
-    sym_to_parent<u>(t[u], q, c.b);
+    sym_to_parent<u, false>(t[u], q, c.b);
     add_sym_outer<S>(S(0.5), S(r[0]), S(r[1]), S(r[2]), c.p, c.b);
     for (int i = 0; i < 6; ++i) c.b[i] += B[i];
     to_parent_add<u>(t[u], c.n, h, c.n);
