@@ -12,6 +12,7 @@
 
 #include "batch_kernels.hpp"
 #include "context.hpp"
+#include "slot_wait.hpp"
 
 using namespace rbdi;
 
@@ -34,6 +35,7 @@ struct rbd_batch {
   char* dh_stage[kRing] = {};         // their device addresses
   hipEvent_t staged[kRing] = {};      // a slot's copy has read it, or
   uint64_t read_seq[kRing] = {};      // the word in the slot that its staging kernel sets (0: none pending)
+  hipStream_t read_on[kRing] = {};    // and the stream that kernel is on
   uint64_t next_seq = 0;
   int ring = 0;
   // persistent grid per shape, and the captured graphs per (shape, small
@@ -290,14 +292,34 @@ void stage_prefix(char* dst, int n_traj) {
 
 uint64_t* read_word(char* slot) { return reinterpret_cast<uint64_t*>(slot + kReadWord); }
 
-// Until the last batch staged in slot r has been read out of it.
+// Whether work issued to stream s may still be running; *err: what has become
+// of it, if not.  A stream under capture cannot be asked (its earlier work runs
+// on), and a handle that the runtime does not know (the caller has destroyed
+// the stream) says nothing: then the device's work is waited for.
+bool stream_pending(hipStream_t s, int* err) {
+  hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+  hipError_t e = hipStreamIsCapturing(s, &capturing);
+  if (e == hipSuccess && capturing == hipStreamCaptureStatusNone) e = hipStreamQuery(s);
+  const bool under_capture = capturing != hipStreamCaptureStatusNone ||
+                             (e >= hipErrorStreamCaptureUnsupported && e <= hipErrorStreamCaptureWrongThread);
+  if (e != hipSuccess && e != hipErrorNotReady && !under_capture) e = hipDeviceSynchronize();
+  (void)hipGetLastError();              // "not ready" is no launch's error
+  if (under_capture || e == hipErrorNotReady) return true;
+  *err = int(e);
+  return false;
+}
+
+// Until the last batch staged in slot r has been read out of it, or has failed.
 hipError_t wait_slot(rbd_batch* b, int r) {
   const uint64_t seq = b->read_seq[r];
   if (seq == 0) return hipEventSynchronize(b->staged[r]);
-  for (int spins = 0; __atomic_load_n(read_word(b->h_stage[r]), __ATOMIC_ACQUIRE) != seq; ++spins)
-    if (spins > (1 << 12)) std::this_thread::yield();       // the stream is four batches behind
-  b->read_seq[r] = 0;
-  return hipSuccess;
+  const uint64_t* word = read_word(b->h_stage[r]);
+  const int e = wait_for_word([&] { return __atomic_load_n(word, __ATOMIC_ACQUIRE) == seq; },
+                              [] { std::this_thread::yield(); },
+                              [&](int* err) { return stream_pending(b->read_on[r], err); },
+                              int(hipErrorLaunchFailure));
+  if (e == 0) b->read_seq[r] = 0;
+  return hipError_t(e);
 }
 
 int graph_index(Shape sh, bool small) { return 2 * mapping_of(sh) + (small ? 1 : 0); }
@@ -538,6 +560,7 @@ rbd_status rbdi::batch_run(rbd_batch* b, const rbd_traj* trajs, int n_traj, int 
     e = hipGetLastError();
     if (e != hipSuccess) return hip_fail(e, "batch staging kernel");
     b->read_seq[r] = seq;
+    b->read_on[r] = st;
     Queue q = own_queue(b);
     q.chunks = chunks;
     q.planned = true;
