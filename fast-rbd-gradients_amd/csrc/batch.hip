@@ -261,20 +261,40 @@ hipError_t launch_batch(rbd_batch* b, const Queue& q, Shape sh, bool small, hipS
   }
 }
 
+rbd::TrajDesc descriptor(const rbd_traj& t) { return rbd::TrajDesc{t.d_in, t.d_out, long(t.n_knots), 0}; }
+
+rbd::BatchHeader header(const rbd_traj* trajs, int n_traj, int lanes) {
+  rbd::BatchHeader h{};
+  h.n_traj = n_traj;
+  // the plan kernel's prefix sum counts chunks of this many knots per
+  // trajectory: single knots for the L-lane groups, whose chunks cross trajectories
+  h.chunk_knots = is_group_lanes(lanes) ? 1 : int(chunk_knots(lanes));
+  h.total_chunks = long(chunk_total(n_traj, [trajs](int t) { return int64_t(trajs[t].n_knots); }, lanes));
+  return h;
+}
+
 // header + descriptors of a batch into host memory at dst (kHeaderBytes, then
 // the descriptors); returns the chunk total
 long stage(char* dst, const rbd_traj* trajs, int n_traj, int lanes) {
   rbd::BatchHeader* h = reinterpret_cast<rbd::BatchHeader*>(dst);
-  std::memset(h, 0, sizeof(*h));
+  *h = header(trajs, n_traj, lanes);
   rbd::TrajDesc* d = reinterpret_cast<rbd::TrajDesc*>(dst + kHeaderBytes);
-  for (int t = 0; t < n_traj; ++t) d[t] = rbd::TrajDesc{trajs[t].d_in, trajs[t].d_out, long(trajs[t].n_knots), 0};
-  const long total = long(chunk_total(n_traj, [trajs](int t) { return int64_t(trajs[t].n_knots); }, lanes));
-  h->n_traj = n_traj;
-  // the plan kernel's prefix sum counts chunks of this many knots per
-  // trajectory: single knots for the L-lane groups, whose chunks cross trajectories
-  h->chunk_knots = is_group_lanes(lanes) ? 1 : int(chunk_knots(lanes));
-  h->total_chunks = total;
-  return total;
+  for (int t = 0; t < n_traj; ++t) d[t] = descriptor(trajs[t]);
+  return h->total_chunks;
+}
+
+// header + descriptors of a batch to the batch's device memory through kernel
+// arguments (batch_args_kernel), for a stream under capture
+hipError_t upload_in_arguments(rbd_batch* b, const rbd_traj* trajs, int n_traj, const rbd::BatchHeader& h,
+                               hipStream_t st) {
+  for (int first = 0; first < n_traj; first += rbd::kSmallBatch) {
+    rbd::ArgBatch a{};
+    a.n_traj = n_traj - first < rbd::kSmallBatch ? n_traj - first : rbd::kSmallBatch;
+    for (int t = 0; t < a.n_traj; ++t) a.d[t] = descriptor(trajs[first + t]);
+    hipLaunchKernelGGL(rbd::batch_args_kernel, dim3(1), dim3(rbd::kSmallBatch), 0, st, a, first, h, b->d_desc, b->d_hdr);
+    if (const hipError_t e = hipGetLastError()) return e;
+  }
+  return hipSuccess;
 }
 
 // The prefix sum the plan kernel would make, behind the staged descriptors
@@ -535,49 +555,49 @@ rbd_status rbdi::batch_run(rbd_batch* b, const rbd_traj* trajs, int n_traj, int 
     if (le != hipSuccess) return hip_fail(le, "batch kernel launch");
     return RBD_OK;
   }
-  // stage header and descriptors in pinned memory, from where a kernel or a
-  // copy on `stream` takes them; a stream under capture records the copy, since
-  // its kernel would set the slot's word only when the graph runs
-  const int r = b->ring;
-  b->ring = (r + 1) % rbd_batch::kRing;
-  hipError_t e = wait_slot(b, r);     // the previous batch has been read out of this slot
-  if (e != hipSuccess) return hip_fail(e, "staging wait");
-  const int64_t chunks = stage(b->h_stage[r], trajs, n_traj, lanes);
   hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-  if (!use_graph && n_traj <= rbd::kStageTrajectories) {
-    e = hipStreamIsCapturing(st, &capturing);
-    if (e != hipSuccess) return hip_fail(e, "stream status");
+  hipError_t e = hipStreamIsCapturing(st, &capturing);
+  if (e != hipSuccess) return hip_fail(e, "stream status");
+  Queue q = own_queue(b);
+  if (capturing != hipStreamCaptureStatusNone) {
+    // a graph that replays this call must not read a staging slot: later calls reuse it
+    const rbd::BatchHeader h = header(trajs, n_traj, lanes);
+    q.chunks = h.total_chunks;
+    e = upload_in_arguments(b, trajs, n_traj, h, st);
+    if (e != hipSuccess) return hip_fail(e, "batch descriptor kernel");
+  } else {
+    // stage header and descriptors in pinned memory, from where a kernel or a
+    // copy on `stream` takes them
+    const int r = b->ring;
+    b->ring = (r + 1) % rbd_batch::kRing;
+    e = wait_slot(b, r);                // the previous batch has been read out of this slot
+    if (e != hipSuccess) return hip_fail(e, "staging wait");
+    q.chunks = stage(b->h_stage[r], trajs, n_traj, lanes);
+    if (!use_graph && n_traj <= rbd::kStageTrajectories) {
+      stage_prefix(b->h_stage[r], n_traj);
+      char* d_slot = b->dh_stage[r];
+      const uint64_t seq = ++b->next_seq;
+      hipLaunchKernelGGL(rbd::batch_stage_kernel, dim3(1), dim3(rbd::kPlanThreads), 0, st,
+                         reinterpret_cast<const rbd::v4i*>(d_slot + kHeaderBytes),
+                         *reinterpret_cast<const rbd::BatchHeader*>(b->h_stage[r]),
+                         reinterpret_cast<rbd::v4i*>(b->d_desc), b->d_hdr, reinterpret_cast<rbd::v4i*>(b->d_prefix),
+                         reinterpret_cast<unsigned long long*>(d_slot + kReadWord), (unsigned long long)seq);
+      e = hipGetLastError();
+      if (e != hipSuccess) return hip_fail(e, "batch staging kernel");
+      b->read_seq[r] = seq;
+      b->read_on[r] = st;
+      q.planned = true;
+    } else {
+      e = hipMemcpyAsync(b->d_mem, b->h_stage[r], batch_stage_bytes(n_traj), hipMemcpyHostToDevice, st);
+      if (e == hipSuccess) e = hipEventRecord(b->staged[r], st);
+      if (e != hipSuccess) return hip_fail(e, "descriptor upload");
+    }
   }
-  if (!use_graph && n_traj <= rbd::kStageTrajectories && capturing == hipStreamCaptureStatusNone) {
-    stage_prefix(b->h_stage[r], n_traj);
-    char* d_slot = b->dh_stage[r];
-    const uint64_t seq = ++b->next_seq;
-    hipLaunchKernelGGL(rbd::batch_stage_kernel, dim3(1), dim3(rbd::kPlanThreads), 0, st,
-                       reinterpret_cast<const rbd::v4i*>(d_slot + kHeaderBytes),
-                       *reinterpret_cast<const rbd::BatchHeader*>(b->h_stage[r]),
-                       reinterpret_cast<rbd::v4i*>(b->d_desc), b->d_hdr, reinterpret_cast<rbd::v4i*>(b->d_prefix),
-                       reinterpret_cast<unsigned long long*>(d_slot + kReadWord), (unsigned long long)seq);
-    e = hipGetLastError();
-    if (e != hipSuccess) return hip_fail(e, "batch staging kernel");
-    b->read_seq[r] = seq;
-    b->read_on[r] = st;
-    Queue q = own_queue(b);
-    q.chunks = chunks;
-    q.planned = true;
-    e = launch_batch(b, q, sh, small, st);
-    if (e != hipSuccess) return hip_fail(e, "batch kernel launch");
-    return RBD_OK;
-  }
-  e = hipMemcpyAsync(b->d_mem, b->h_stage[r], batch_stage_bytes(n_traj), hipMemcpyHostToDevice, st);
-  if (e == hipSuccess) e = hipEventRecord(b->staged[r], st);
-  if (e != hipSuccess) return hip_fail(e, "descriptor upload");
   if (use_graph) {
     if (rbd_status s = ensure_graph(b, sh, small)) return s;
     e = hipGraphLaunch(b->exec[graph_index(sh, small)], st);
     if (e != hipSuccess) return hip_fail(e, "hipGraphLaunch");
   } else {
-    Queue q = own_queue(b);
-    q.chunks = chunks;
     e = launch_batch(b, q, sh, small, st);
     if (e != hipSuccess) return hip_fail(e, "batch kernel launch");
   }

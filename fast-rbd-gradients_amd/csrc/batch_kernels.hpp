@@ -147,6 +147,19 @@ __global__ __launch_bounds__(kPlanThreads) void batch_stage_kernel(const v4i* __
   if (t == 0) __hip_atomic_store(done, seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
+// Part of a list whose call is being captured: up to 64 descriptors, from
+// `first` on, from the kernel's arguments to the batch's device memory, and the
+// header with the first of them.  A graph keeps its kernels' arguments, so every
+// replay brings the captured list; a staging slot would by then hold a later
+// call's.  (A captured list of 4,097 trajectories is 65 such nodes.)
+__global__ __launch_bounds__(kSmallBatch) void batch_args_kernel(ArgBatch a, int first, BatchHeader h,
+                                                                 TrajDesc* __restrict__ descs,
+                                                                 BatchHeader* __restrict__ hdr) {
+  const int t = int(threadIdx.x);
+  if (t < a.n_traj) descs[first + t] = a.d[t];
+  if (first == 0 && t == 0) *hdr = h;
+}
+
 // The largest t below n with prefix[t] <= key (prefix[0] <= key), by the whole
 // wave: 64 places at a time, so two dependent loads for up to 4,096
 // trajectories where halving takes up to 12.

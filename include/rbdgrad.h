@@ -326,7 +326,10 @@ rbd_status rbd_batch_destroy(rbd_batch* b);
 /* Run the forward-dynamics gradient over n_traj trajectories on `stream`.
  * Up to 64 trajectories travel in the kernel's arguments (no upload); more
  * are copied to the device asynchronously on `stream`.  The caller's trajs
- * array may be reused on return.  The knot-to-lane mapping is chosen from the
+ * array may be reused on return.  A call on a stream under capture is recorded
+ * with its list: every replay of the caller's graph runs that list, whatever
+ * the batch object has run since (replays and calls on it stay in one stream's
+ * order).  The knot-to-lane mapping is chosen from the
  * total knot count by the context's batch mapping table (rbd_autotune_batch),
  * unless the context fixes lanes_per_knot (32: the two-wave mapping, 4-knot
  * chunks on workgroups of two waves; 4, 7, 8: chunks of 16, 9, 8 knots of the
