@@ -130,7 +130,10 @@ RBD_HD RBD_INLINE void sincos_reduced(double x, double* s, double* c) {
 // (Payne and Hanek's reduction): with x = m 2^E, the bits of 2/pi from weight
 // 2^(1 - E) on, as a 128-bit number W, give x 2/pi mod 4 = (m W mod 2^128)
 // 2^-126: two bits of quadrant and 126 of fraction, of which an FP32 x cancels
-// at most about 30.
+// at most about 30.  For FP64 results (S) the fraction is taken in two words
+// and multiplied by pi/2 in two, so that r is rounded once and the results stay
+// within 2 units in the last place (one word of each: 2.6).
+template <typename S>
 RBD_HD RBD_INLINE void sincos_far(float x, double* s, double* c) {
   constexpr unsigned kTwoOverPi[9] = {0u, 0xa2f9836eu, 0x4e441529u, 0xfc2757d1u, 0xf534ddc0u, 0xdb629599u, 0x3c439041u, 0xfe5163abu, 0xdebbc561u};
   const unsigned bits = __builtin_bit_cast(unsigned, x);
@@ -157,8 +160,16 @@ RBD_HD RBD_INLINE void sincos_far(float x, double* s, double* c) {
   const unsigned long long hi = (static_cast<unsigned long long>(limb[0]) << 32) | limb[1];
   const unsigned long long lo = (static_cast<unsigned long long>(limb[2]) << 32) | limb[3];
   const unsigned q = unsigned((hi + (1ull << 61)) >> 62);           // nearest quarter turn
-  const double f = double(static_cast<long long>(hi - (static_cast<unsigned long long>(q) << 62))) + double(lo) * 0x1p-64;
-  const double r = f * (0x1p-62 * 0x1.921fb54442d18p+0);
+  const long long whole = static_cast<long long>(hi - (static_cast<unsigned long long>(q) << 62));
+  constexpr double half_pi = 0x1p-62 * 0x1.921fb54442d18p+0, half_pi_low = 0x1p-62 * 0x1.1a62633145c07p-54;
+  double r;
+  if constexpr (sizeof(S) == 8) {
+    const double f = double(whole);
+    const double low = double(whole - static_cast<long long>(f)) + double(lo) * 0x1p-64;
+    r = __builtin_fma(f, half_pi, __builtin_fma(low, half_pi, f * half_pi_low));
+  } else {
+    r = (double(whole) + double(lo) * 0x1p-64) * half_pi;
+  }
   const bool neg = (bits >> 31) != 0u;
   sincos_quadrant(neg ? 0u - q : q, neg ? -r : r, s, c);
 }
@@ -170,7 +181,7 @@ RBD_HD RBD_INLINE void sincos_s(S x, S* s, S* c) {
   const bool far = !(__builtin_fabs(x) <= kSincosMax<S>);
   if (__ballot(far) != 0) {              // the same in every lane
     double sf, cf;
-    sincos_far(float(x), &sf, &cf);
+    sincos_far<S>(float(x), &sf, &cf);
     *s = far ? S(sf) : *s;
     *c = far ? S(cf) : *c;
   }
