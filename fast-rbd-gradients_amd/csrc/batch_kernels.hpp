@@ -9,8 +9,10 @@
 //   * up to 64 trajectories (SMALL): a wave scans the counts itself, one
 //     trajectory per lane, and finds the chunk's trajectory with a ballot and
 //     a population count -- no plan kernel, no memory traffic beyond the counts;
-//   * more: the plan kernel writes the prefix sum first, and the waves
-//     binary-search it.
+//   * more: the waves search the prefix sum in memory, 64 places at a time.
+//     The host forms it beside the list (up to kStageTrajectories, which one
+//     kernel stages) or the plan kernel does (longer lists, graph replays,
+//     calls under capture).
 // With G waves in the grid and T chunks, the waves pull the chunks of the full
 // rounds, floor(T / G) * G of them, in a fixed order (wave w: w, w + G, ...),
 // which needs no atomic: every chunk costs the same, so a fixed order is
@@ -69,7 +71,7 @@ struct Completion {
   unsigned long long seq;
 };
 
-constexpr int kSmallBatch = 64;   // trajectories handled without the plan kernel
+constexpr int kSmallBatch = 64;   // trajectories handled without a prefix sum in memory
 
 // A small batch passed by value in the kernel arguments, so that a direct
 // launch needs no descriptor upload; used when descs is null.

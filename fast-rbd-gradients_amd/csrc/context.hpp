@@ -19,13 +19,13 @@ constexpr int kBlock = 64;   // one wave per workgroup (the 4-, 7- and 8-lane gr
 // With the thresholds deciding (a threshold set by hand drops the mapping
 // table), calls of up to this many knots use the 16-lane-group mapping
 // instead of one lane per knot: the crossover measured on MI355X (one-lane
-// 10.6 us vs lane-group 8.9 us at 8,192 knots, 10.6 vs 13.2 us at 9,216).
+// 9.6 us vs lane-group 8.9 us at 8,192 knots, 9.6 vs 13.3 us at 9,216).
 constexpr int64_t kDefaultGroupThreshold = 8192;
 // The two-wave mapping (Minv and the RNEA + columns of a knot on two waves)
 // serves calls up to the context's two_wave_threshold knots: by default
 // 16 x compute units (4,096 knots on 256 CUs, the crossover rbd_autotune
-// measured on MI355X: 5.95 us against 7.55 us for one-wave lane groups at 4,096
-// knots, 12.2 against 8.9 us at 8,192); rbd_autotune measures it.
+// measured on MI355X: 5.97 us against 7.50 us for one-wave lane groups at 4,096
+// knots, 12.4 against 8.9 us at 8,192); rbd_autotune measures it.
 constexpr int kTwoWaveLanes = 32;   // lanes_per_knot value of the two-wave mapping (16 lanes in each of 2 waves)
 // lanes_per_knot values of the L-lane groups of group_mapping.hpp (full path only)
 inline bool is_group_lanes(int lanes) { return lanes == 4 || lanes == 7 || lanes == 8; }
@@ -33,9 +33,8 @@ inline bool is_group_lanes(int lanes) { return lanes == 4 || lanes == 7 || lanes
 // parameter; the waves of a workgroup share nothing).  Larger workgroups put
 // one wave on each SIMD of a CU, which the dispatcher does not do for
 // single-wave workgroups; at about one wave per SIMD (9,216 knots in 7-lane
-// groups) the sizes measure within 1-2% of each other (7.70 us in workgroups
-// of 4, 7.79 in workgroups of 1).
-constexpr int kMaxWavesPerGroup = rbd::kMaxGroupWaves;
+// groups) the sizes measure within 1-2% of each other (7.90 us in workgroups
+// of 4, 7.92 in workgroups of 1).
 inline bool valid_wpg(int w) { return w == 1 || w == 2 || w == 4; }
 // A knot-to-lane mapping and its workgroup shape.
 struct Shape {
@@ -61,7 +60,7 @@ struct MappingTable {
 };
 // The same crossover for batches (rbd_batch_*, total knots of the batch),
 // measured by rbd_autotune_batch on batches of 132-knot trajectories
-// (6,336 knots on MI355X: one-lane 11.6 us vs lane-group 9.2 us; 11.9 vs 15.4
+// (6,336 knots on MI355X: one-lane 11.3 us vs lane-group 9.2 us; 11.7 vs 15.5
 // us at 8,448).
 constexpr int64_t kDefaultBatchGroupThreshold = 8192;
 // Batches of up to this many trajectories find a chunk's trajectory inside the
@@ -141,10 +140,10 @@ constexpr int kAutotuneSizes = 12;
 // groups of 4 lanes up to one wave of 16 (16,384), then one lane per knot;
 // per batch the same without the two-wave mapping, whose looping batch kernel
 // trails the groups of 7 lanes there.
-// (Measured: a call of 4,096 knots 5.95 us with two waves, 7.3 with 7 lanes;
-// 9,216 knots 7.7 us with 7 lanes, 8.8 with 4, 10.6 with one; 16,384 knots 10.2
-// with 4, 10.9 with one; 24,576 knots 17.0 with 4, 11.4 with one; a batch of 64
-// trajectories of 142 knots 8.9 us with 7 lanes, 9.9 with 4, 14.7 with one.)
+// (Measured: a call of 4,096 knots 5.97 us with two waves, 7.4 with 7 lanes;
+// 9,216 knots 7.9 us with 7 lanes, 8.7 with 4, 9.6 with one; 16,384 knots 10.1
+// with 4, 10.0 with one; 24,576 knots 17.0 with 4, 10.5 with one; a batch of 64
+// trajectories of 142 knots 9.05 us with 7 lanes, 9.9 with 4, 11.5 with one.)
 inline void set_default_tables(rbd_context* ctx) {
   const int64_t simds = 4 * int64_t(ctx->compute_units);
   const int64_t n[4] = {4 * simds, 9 * simds, 16 * simds, INT64_MAX};

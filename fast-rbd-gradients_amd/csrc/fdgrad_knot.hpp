@@ -132,7 +132,7 @@ RBD_HD RBD_INLINE void sincos_reduced(double x, double* s, double* c) {
 // 2^-126: two bits of quadrant and 126 of fraction, of which an FP32 x cancels
 // at most about 30.  For FP64 results (S) the fraction is taken in two words
 // and multiplied by pi/2 in two, so that r is rounded once and the results stay
-// within 2 units in the last place (one word of each: 2.6).
+// within 2 units in the last place (1.50; one word of each: 2.53).
 template <typename S>
 RBD_HD RBD_INLINE void sincos_far(float x, double* s, double* c) {
   constexpr unsigned kTwoOverPi[9] = {0u, 0xa2f9836eu, 0x4e441529u, 0xfc2757d1u, 0xf534ddc0u, 0xdb629599u, 0x3c439041u, 0xfe5163abu, 0xdebbc561u};
@@ -231,11 +231,11 @@ RBD_HD RBD_INLINE void xmotion(const CS<S>& t, const S* x, S* y) {
   y[0] = y0[0]; y[1] = y0[1]; y[2] = y0[2];
   y[3] = y1[0]; y[4] = y1[1]; y[5] = y1[2];
 }
-// y = T^T x (+ z) for a force vector: [E^T n + r x (E^T f); E^T f] (+ z).
-// The angular rows add each product to the row on its own (one FMA each),
-// starting from z when there is one.
-template <int K, bool ADD, typename S>
-RBD_HD RBD_INLINE void xforce_t_into(const CS<S>& t, const S* x, const S* z, S* y) {
+// y = T^T x + z for a force vector: [E^T n + r x (E^T f); E^T f] + z.  The
+// angular rows add each product to the row on its own (one FMA each), starting
+// from z.
+template <int K, typename S>
+RBD_HD RBD_INLINE void xforce_t_add(const CS<S>& t, const S* x, const S* z, S* y) {
   constexpr S rx = roff<K, S>(0), ry = roff<K, S>(1), rz = roff<K, S>(2);
   S fl[3];
   rot_t<K>(t, x + 3, fl);
@@ -243,7 +243,7 @@ RBD_HD RBD_INLINE void xforce_t_into(const CS<S>& t, const S* x, const S* z, S* 
   static_for<0, 3>([&](auto Jc) {
     constexpr int j = decltype(Jc)::value;
     constexpr int j1 = (j + 1) % 3, j2 = (j + 2) % 3;
-    S acc = ADD ? z[j] : S(0);
+    S acc = z[j];
     acc += Eij<K, 0, j>(t) * x[0];
     acc += Eij<K, 1, j>(t) * x[1];
     acc += Eij<K, 2, j>(t) * x[2];
@@ -251,16 +251,7 @@ RBD_HD RBD_INLINE void xforce_t_into(const CS<S>& t, const S* x, const S* z, S* 
     acc -= r[j2] * fl[j1];
     y[j] = acc;
   });
-  for (int j = 0; j < 3; ++j) y[3 + j] = ADD ? z[3 + j] + fl[j] : fl[j];
-}
-template <int K, typename S>
-RBD_HD RBD_INLINE void xforce_t(const CS<S>& t, const S* x, S* y) {
-  xforce_t_into<K, false>(t, x, static_cast<const S*>(nullptr), y);
-}
-// y = T^T x + z
-template <int K, typename S>
-RBD_HD RBD_INLINE void xforce_t_add(const CS<S>& t, const S* x, const S* z, S* y) {
-  xforce_t_into<K, true>(t, x, z, y);
+  for (int j = 0; j < 3; ++j) y[3 + j] = z[3 + j] + fl[j];
 }
 
 // entry (R, C) of link K's spatial inertia, as a compile-time constant
@@ -280,7 +271,7 @@ RBD_HD RBD_INLINE void imv(const S* x, S* y) {
     y[r] = ACC ? y[r] + acc : acc;
   });
 }
-// A = I_K
+// A = I_K (for the host's check of the model's tables)
 template <int K, typename S>
 RBD_HD RBD_INLINE void iload(S A[6][6]) {
   static_for<0, 6>([&](auto Rc) {
@@ -565,18 +556,18 @@ using PrecFP64      = Precision<double, double, double, double>; // all FP64
 // RNEA and columns a knot's state fits in 256 registers per lane, so two waves
 // share a SIMD: a wave issues at most one instruction every 4 cycles, so two
 // issue twice as many (and each hides the other's latency); with FP64 columns
-// it needs about 500 and runs one.
+// it needs 320 to 500 and runs one.
 template <class P>
 constexpr int kWavesPerSimd = (sizeof(typename P::Col) == 4 && sizeof(typename P::Rnea) == 4) ? 2 : 1;
 
-// sin/cos of a joint angle under precision P: the math library's sincos, or,
-// with P::kHwTrig and an FP32 angle, the hardware's v_sin_f32/v_cos_f32 (whose
-// argument is in revolutions).  The angle is first reduced to [-pi, pi] as
+// sin/cos of a joint angle under precision P: sincos_s, or, with P::kHwTrig and
+// an FP32 angle, the hardware's v_sin_f32/v_cos_f32 (whose argument is in
+// revolutions).  The angle is first reduced to [-pi, pi] as
 // x - k 2pi with 2pi split into two FP32 parts (exact to about 2^-40 |x|), so
-// small and large angles keep their precision.  Measured on MI355X: 2% less
-// per-call latency at 128 knots and 1% less time at 2^20 knots, and the
-// largest relative output error over 2^20 random and stretched-arm poses
-// 6.5e-5 instead of 4.1e-5.  The host build uses the math library's.
+// small and large angles keep their precision.  Measured on MI355X: a call of
+// 128 knots 4.37 us against 4.49, 2^20 knots 100.0 against 101.2, and the largest
+// relative output error over 2^20 random and stretched-arm poses 4.5e-5 instead
+// of 1.7e-5.  The host build uses the math library's in both.
 template <class P, typename S>
 RBD_HD RBD_INLINE void knot_sincos(S x, S* s, S* c) {
 #if defined(__HIP_DEVICE_COMPILE__)

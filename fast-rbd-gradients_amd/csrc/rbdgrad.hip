@@ -181,8 +181,11 @@ __global__ __launch_bounds__(kBlock, kWavesPerSimd<P>) void fdgrad_refmode_kerne
 // low-latency mapping for small batches.  Every lane of a group runs the
 // shared steps, then one derivative column; the group's lanes finish together.
 // W: waves per SIMD the kernel is compiled for.  W = 1 lets the compiler use
-// up to 512 registers (no spills: the latency variant, for calls whose waves
-// do not outnumber the SIMDs); W = kWavesPerSimd<P> is the throughput variant.
+// up to 512 registers (the latency variant, for calls whose waves do not
+// outnumber the SIMDs); W = kWavesPerSimd<P> is the throughput variant.  The
+// iiwa's fit in 256 either way and come out the same (252 array of structures,
+// 246 structure of arrays); a robot with dense joint frames needs more (the
+// synthetic arm 288, of which two waves spill 31).
 template <class P, int W>
 __global__ __launch_bounds__(kBlock, W) void fdgrad_aos_lanes_kernel(long n, const float* __restrict__ in,
                                                                   float* __restrict__ out, Options opt) {
@@ -637,9 +640,9 @@ void launch_lanes(const FlatCall& c, dim3 grid, dim3 block) {
 }
 
 // Workgroups (one wave each) of a one-lane kernel that a CU keeps resident,
-// asked of the runtime once per kernel: 8 for the FP32-column SoA kernel (two
-// waves per SIMD), 6 for the array-of-structures one (its LDS record block),
-// 4 for the kernels that stage two output blocks.
+// asked of the runtime once per kernel: 8 with FP32 columns (two waves per
+// SIMD, 13,440 to 19,712 bytes of LDS each), 4 with FP64 columns; the finish
+// kernel 6 (25,088 bytes).
 template <auto Kernel>
 hipError_t resident_per_cu(int* per_cu) {
   static std::atomic<int> cached{0};
@@ -655,9 +658,10 @@ hipError_t resident_per_cu(int* per_cu) {
 
 // A one-lane launch of more 64-knot blocks than the device keeps resident
 // runs one round of resident waves, each looping over blocks w, w + G, ...
-// instead of dispatching a new wave per block: at 2^20 knots 157 against 160
-// us (structure of arrays) and 176 against 183 us (array of structures, whose
-// last round of dispatched waves left SIMDs idle).  cus: the device's compute
+// instead of dispatching a new wave per block, so that a block's loads can go
+// out before the last one's stores.  Both take the same time at 2^20 knots,
+// where memory is the bound (100.9 against 101.2 us structure of arrays, 104.1
+// against 103.4 array of structures).  cus: the device's compute
 // units (0: unknown, the grid stays as it is).
 template <auto Kernel>
 hipError_t one_lane_grid(int cus, dim3* grid) {

@@ -14,8 +14,6 @@
 
 namespace rbd {
 
-constexpr int kRecordBlockFloats = 64 * kOutPerKnot;   // one wave's records
-
 // A store that the caches treat as streaming (non-temporal) when NT: the
 // outputs are written once and not read again by the kernel.
 template <bool NT, typename T>
@@ -113,9 +111,11 @@ __device__ RBD_INLINE void put_block(const BlockPieces<F>& b, int words, int lan
 }
 
 // Whether a one-lane kernel of precision P keeps a knot's outputs in registers
-// until they are complete: with FP32 columns they fit (255 registers, no
-// spills, two waves per SIMD: what the derivative pass no longer needs makes
-// room for them); with FP64 columns they go into LDS as they come.
+// until they are complete: with FP32 columns they fit in the 256 registers of
+// two waves per SIMD (what the derivative pass no longer needs makes room for
+// them; the iiwa's array-of-structures kernel 253 and none spilled, external
+// forces 1 spilled, the 147 floats of the WAFR layout 23; the synthetic arm's
+// kernels 34 to 53); with FP64 columns they go into LDS as they come.
 template <class P> constexpr bool kHoldOutputs = kWavesPerSimd<P> == 2;
 // Floats of LDS for records of REC floats
 template <class P, int REC> constexpr int kRecordLds = (kHoldOutputs<P> ? 32 : 64) * REC;
